@@ -51,11 +51,11 @@ struct gpugi_ctx {
   void* dCounters = nullptr;  // [0] ray counter, [1] error flag, [2] hit count
   void* dWideQueue = nullptr;  // the wide trace kernel's batch counters
   size_t spillBytes = 0;
-  uint32_t wideMaxStack = 0;
+  uint32_t wideMaxStack = 0, wideMaxPending = 0;
   int wideLeaf = 2;     // triangles per merged wide leaf
   int wideStack = 10;   // LDS stack entries per lane of the trace kernel
   int wideRefill = 8;   // idle lanes that trigger a wave-level ray refill
-  int wideWait = 16;    // lanes waiting with a pending leaf that trigger a leaf pass
+  int wideWait = 8;     // lanes waiting with a pending leaf that trigger a leaf pass
   // host copy of the reference layout (re-packing after a configuration change)
   std::vector<float> hHier, hPos;
   std::vector<int32_t> hTris;
@@ -262,6 +262,7 @@ int RebuildWide(gpugi_ctx* ctx) {
     HIP_TRY(ctx, hipMemcpy(ctx->dWideTris, wide.tris.data(), wide.tris.size() * sizeof(WideTriHost),
                            hipMemcpyHostToDevice));
   ctx->wideMaxStack = wide.maxStack;
+  ctx->wideMaxPending = wide.maxPending;
   ctx->hasWide = true;
   return GPUGI_OK;
 }
@@ -1364,7 +1365,7 @@ int gpugi_get_wide_config(gpugi_ctx* ctx, int* max_leaf_triangles, int* lds_stac
   if (lds_stack_entries) *lds_stack_entries = ctx->wideStack;
   if (refill_lanes) *refill_lanes = ctx->wideRefill;
   if (wait_lanes) *wait_lanes = ctx->wideWait;
-  if (max_stack) *max_stack = ctx->wideMaxStack;
+  if (max_stack) *max_stack = ctx->wideMaxPending;
   return GPUGI_OK;
 }
 

@@ -1,28 +1,36 @@
-// Ordered traversal of the 4-wide quantized BVH (wide_bvh.h), one ray per lane.
+// Ordered traversal of the 8-wide quantized BVH (wide_bvh.h), one ray per lane.
 //
-// A ray's state holds the next inner node to visit, up to two pending leaves
-// and a stack of (child word, entry distance) pairs.  Work comes in two kinds
-// of wave-wide passes:
-//   box pass   every lane with a node visits it: four child box tests, the
-//              nearest hit inner child becomes the next node, the nearest hit
-//              leaf takes a free pending slot, the other hit children are
-//              pushed farthest first;
-//   leaf pass  every lane with pending leaves tests their triangles.
+// A ray's state holds the next inner node to visit, up to two pending leaf
+// groups and a stack.  Work comes in two kinds of wave-wide passes:
+//   box pass   every lane with a node visits it: eight child box tests; the
+//              nearest hit child, if inner, becomes the next node, the other hit
+//              inner children wait together in one stack entry; the hit leaves
+//              take a free pending slot, as one group;
+//   leaf pass  every lane with pending leaves tests the triangles of one.
 // A lane with a pending leaf keeps traversing (speculative traversal,
 // Aila and Laine 2009, "Understanding the efficiency of ray traversal on
 // GPUs"), so a wave runs a leaf pass only once enough lanes wait for one and
 // does not pay a divergent triangle loop on every node visit.  The caller
 // chooses the pass from two ballots (wide_choose_leaf_pass).  Lanes left
-// without a node pop: entries beyond the current hit are dropped, a leaf
-// entry fills a free pending slot, an inner entry becomes the next node.
+// without a node pop: entries whose children all lie beyond the current hit are
+// dropped, a leaf entry fills a free pending slot, a node entry gives its next
+// child and stays until it is empty.
 // The result does not depend on the order of the work: the closest hit is the
 // minimum distance, ties resolved to the smaller reference slot index (the
 // triangle the reference's preorder walk meets first).
 //
-// Per lane, the first S stack entries live in LDS laid out [depth][thread],
-// so lanes at different depths touch different banks; deeper entries spill to
-// global memory (WideStack), sized by the host from the exact worst case of
-// the tree.
+// A stack entry is 8 bytes:
+//   nodes   {firstChild of the parent, waiting | inner << 8 | next << 16 | bound}
+//   leaves  {parent | kWideLeafEntry, waiting | bound}
+// waiting: one bit per slot; next: the slot of the nearest child that waits (the
+// others follow in slot order, smallest box first); bound: the 13 high bits of a
+// float, a lower bound of the waiting children's entry distances.  An any-hit
+// query takes the largest box first, which is the likeliest to hold an occluder,
+// and keeps no distances: next and bound are 0.
+// Per lane, the first S entries live in LDS laid out
+// [depth][thread], so lanes at different depths touch different banks; deeper
+// entries spill to global memory (WideStack), sized by the host from the exact
+// worst case of the tree.
 //
 // Box tests use the quantized boxes the host made conservative, slab distances
 // computed with one fma per plane and a slack that covers their rounding (see
@@ -40,6 +48,8 @@
 namespace gpugi {
 
 constexpr uint32_t kWideNoNode = 0xffffffffu;
+constexpr uint32_t kWideLeafEntry = 0x80000000u;
+constexpr uint32_t kWideBoundMask = 0xfff80000u;
 
 struct WideResult {
   float t;     // final ray length (tmax on a miss)
@@ -48,7 +58,7 @@ struct WideResult {
   bool any;    // any-hit result
 };
 
-// A lane's traversal stack of {child word, entry distance bits}: entry i < S at
+// A lane's traversal stack: entry i < S at
 // LDS lds[i * B + tid], deeper entries at spill[(i - S) * spillStride]
 // (spillStride = number of threads sharing the spill buffer when it is laid out
 // [depth][thread], so a wave's spills at one depth are contiguous; 1 for a
@@ -70,9 +80,6 @@ struct WideStack {
   uint32_t spillStride;
 };
 
-// Pending-leaf slots per lane, filled in order (slot j is taken only while
-// slots 0..j-1 are).
-constexpr int kWidePending = 2;
 
 struct WideState {
   gg::V3 o, d;
@@ -81,7 +88,8 @@ struct WideState {
   int bestSlot;
   float bu, bv;
   uint32_t node;  // next inner node to visit, kWideNoNode if none
-  uint32_t leaf[kWidePending];  // pending leaf child words (leaf flag set), 0 if free
+  uint32_t leafNode[2];  // the pending leaf groups' nodes
+  uint32_t leafMask;     // their hit leaves' slots, 8 bits each; 0: none, below 256: the first only
   int sp;
   bool found;
   WtRay wr;  // watertight mode only
@@ -95,7 +103,25 @@ __device__ __forceinline__ float safe_inv(float d) {
   return __builtin_amdgcn_rcpf(fabsf(d) > tiny ? d : copysignf(tiny, d));
 }
 
-__device__ __forceinline__ float byte_f(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xffu); }
+// Two quantized planes as 16-bit integers: bytes i and i + 1 of `lo` or of `hi`,
+// i = 0 or 2; which word is in the selector (kPlaneLo, kPlaneHi for i = 0).
+constexpr uint32_t kPlaneLo = 0x0c010c00u, kPlaneHi = 0x0c050c04u, kPlaneOther = kPlaneLo ^ kPlaneHi;
+constexpr uint32_t kPlaneNextPair = 0x00020002u;
+__device__ __forceinline__ uint32_t plane_pair(uint32_t lo, uint32_t hi, uint32_t selector) {
+  return __builtin_amdgcn_perm(hi, lo, selector);
+}
+
+// q * A + b for the low (half 0) or high plane q of a pair, A24 = A * 2^24: a byte
+// read as a binary16 is exactly q * 2^-24 (a subnormal), which the mixed-precision
+// fma takes as it is, so no conversion instruction is needed.
+__device__ __forceinline__ float plane_fma(uint32_t pair, int half, float A24, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
+  return __builtin_fmaf((float)__builtin_bit_cast(Half2, pair)[half], A24, b);
+#else
+  return __builtin_fmaf((float)((pair >> (16 * half)) & 0xffffu) * 5.9604644775390625e-8f, A24, b);
+#endif
+}
 
 template <bool WT = false>
 __device__ __forceinline__ void wide_init(WideState& st, gg::V3 o, gg::V3 d, float tmax) {
@@ -108,179 +134,175 @@ __device__ __forceinline__ void wide_init(WideState& st, gg::V3 o, gg::V3 d, flo
   st.bestSlot = -1;
   st.bu = st.bv = 0.0f;
   st.node = 0;
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) st.leaf[j] = 0;
+  st.leafNode[0] = st.leafNode[1] = 0;
+  st.leafMask = 0;
   st.sp = 0;
   st.found = false;
   if (WT) st.wr = wt_setup(d);
 }
 
+// The node in slot `slot` of the node whose inner children (mask `inner`) start at `first`.
+__device__ __forceinline__ uint32_t wide_child(uint32_t first, uint32_t inner, uint32_t slot) {
+  return first + (uint32_t)__popc(inner & ((1u << slot) - 1u));
+}
+
+// Which of the waiting slots (not 0) is visited next: the nearest one if it waits
+// (if it is not a leaf or gone already), else the first; any hit: the last.
+template <bool ANY>
+__device__ __forceinline__ uint32_t wide_next(uint32_t waiting, uint32_t nearest) {
+  if (ANY) return 31u - (uint32_t)__builtin_clz(waiting);
+  return (waiting >> nearest) & 1u ? nearest : (uint32_t)__builtin_ctz(waiting);
+}
+
+// Puts an entry on the stack; false if it would overflow (impossible when the
+// host sized the spill from the tree).
+template <int B, int S>
+__device__ __forceinline__ bool wide_push(const WideScene& s, WideState& st, const WideStack& stk, uint2 e) {
+  if (st.sp < S) stk.lds[st.sp * B + stk.tid] = e;
+  else if ((uint32_t)(st.sp - S) < s.spillDepth) stk.spill[(size_t)(st.sp - S) * stk.spillStride] = e;
+  else return false;
+  ++st.sp;
+  return true;
+}
+
+// Takes a leaf group (leaves != 0) into a free pending slot; false if both are taken.
+__device__ __forceinline__ bool wide_hold(WideState& st, uint32_t node, uint32_t leaves) {
+  if (st.leafMask > 0xffu) return false;
+  const bool empty = st.leafMask == 0u;
+  st.leafNode[0] = empty ? node : st.leafNode[0];
+  st.leafNode[1] = empty ? st.leafNode[1] : node;
+  st.leafMask |= empty ? leaves : leaves << 8;
+  return true;
+}
+
 // Box pass for a lane with st.node != kWideNoNode.  Returns false if the stack
-// would overflow (impossible when the host sized the spill from the tree).
+// would overflow.
 template <bool ANY, int B, int S>
 __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, const WideStack& stk) {
   const gg::V3 o = st.o;
   const uint32_t nodeIndex = st.node;
-  const uint4 q0 = s.nodes[4 * (size_t)nodeIndex + 0];
-  const uint4 q1 = s.nodes[4 * (size_t)nodeIndex + 1];
-  const uint4 q2 = s.nodes[4 * (size_t)nodeIndex + 2];
-  const uint4 q3 = s.nodes[4 * (size_t)nodeIndex + 3];
+  // (n << 6) + (n << 4) is 80 n, below 2^32 for kWideMaxNodes
+  const uint4* n = (const uint4*)((const char*)s.nodes + ((nodeIndex << 6) + (nodeIndex << 4)));
+  const uint4 q0 = n[0], q1 = n[1], q2 = n[2], q3 = n[3], q4 = n[4];
   const float ox = __uint_as_float(q0.x), oy = __uint_as_float(q0.y), oz = __uint_as_float(q0.z);
   const float sx = __uint_as_float((q0.w & 0xffu) << 23);
   const float sy = __uint_as_float(((q0.w >> 8) & 0xffu) << 23);
   const float sz = __uint_as_float(((q0.w >> 16) & 0xffu) << 23);
-  const int nchild = (int)(q0.w >> 24);
   // Slab distances straight from the quantized bytes: along axis a,
   //   t(q) = (origin_a + q * s_a - o_a) / d_a ~ q * A_a + B_a,
   //   A_a = s_a * inv_a (exact: s_a is a power of two),  B_a = (origin_a - o_a) * inv_a.
-  // With inv_a = (1/d_a)(1 + δ), |δ| <= 2^-23 (safe_inv), every exact distance of
-  // the ray is scaled by 1 + δ; beyond that B_a carries two roundings, so near
-  // distances use B_a - e_a and far ones B_a + e_a with e_a = |B_a| * 2^-21; the
-  // byte word giving the near plane (lo or hi) is picked per axis from the sign of
-  // inv_a.  The host checks in extended precision that origin + q * s encloses
-  // every child box, so with the far distance and the hit distance widened by
-  // 1 + 2^-20 (> 1 + 2^-23 + the fma's rounding) a box that holds the closest hit
-  // is never rejected (the same argument as Ize 2013, "Robust BVH ray traversal").
+  // With inv_a = (1/d_a)(1 + δ_a), |δ_a| <= 2^-23 (safe_inv), the exact distances
+  // along an axis are scaled by 1 + δ_a.  Near distances use B_a - |B_a| * 2^-21,
+  // which covers the two roundings of B_a.  Far ones use
+  // B_a + |B_a| * 2^-20 + |A_a| * 2^-12: along every ray into a box, t is at most
+  // |B_a| + 255 |A_a| for each far plane, so this covers the axes' different δ_a
+  // (2^-22 t), the roundings of B_a (2^-23 |B_a|) and those of both fmas (2^-24 t
+  // each).  The bytes giving the near planes (lo or hi) are picked per axis by the
+  // sign of inv_a.  The host checks in extended precision that origin + q * s
+  // encloses every child box, so with the hit distance widened by 1 + 2^-20 a box
+  // that holds the closest hit is never rejected (the argument of Ize 2013,
+  // "Robust BVH ray traversal").
   const float Ax = sx * st.ix, Ay = sy * st.iy, Az = sz * st.iz;
   const float Bx = (ox - o.x) * st.ix, By = (oy - o.y) * st.iy, Bz = (oz - o.z) * st.iz;
-  const float ex = fabsf(Bx) * 4.76837158e-7f, ey = fabsf(By) * 4.76837158e-7f, ez = fabsf(Bz) * 4.76837158e-7f;
-  const float bnx = Bx - ex, bny = By - ey, bnz = Bz - ez;
-  const float bfx = Bx + ex, bfy = By + ey, bfz = Bz + ez;
-  const uint32_t nearX = st.ix >= 0.0f ? q2.x : q2.w, farX = st.ix >= 0.0f ? q2.w : q2.x;
-  const uint32_t nearY = st.iy >= 0.0f ? q2.y : q3.x, farY = st.iy >= 0.0f ? q3.x : q2.y;
-  const uint32_t nearZ = st.iz >= 0.0f ? q2.z : q3.y, farZ = st.iz >= 0.0f ? q3.y : q2.z;
+  constexpr float kNearSlack = 4.76837158e-7f, kFarSlack = 9.53674316e-7f, kQuantumSlack = 2.44140625e-4f;
+  const float bnx = __builtin_fmaf(-fabsf(Bx), kNearSlack, Bx), bny = __builtin_fmaf(-fabsf(By), kNearSlack, By),
+              bnz = __builtin_fmaf(-fabsf(Bz), kNearSlack, Bz);
+  const float bfx = __builtin_fmaf(fabsf(Ax), kQuantumSlack, __builtin_fmaf(fabsf(Bx), kFarSlack, Bx)),
+              bfy = __builtin_fmaf(fabsf(Ay), kQuantumSlack, __builtin_fmaf(fabsf(By), kFarSlack, By)),
+              bfz = __builtin_fmaf(fabsf(Az), kQuantumSlack, __builtin_fmaf(fabsf(Bz), kFarSlack, Bz));
+  constexpr float k2p24 = 16777216.0f;
+  const float Ax24 = Ax * k2p24, Ay24 = Ay * k2p24, Az24 = Az * k2p24;
   const float tbScaled = st.tbest * 1.00000095f;
-  float tn[4];
+  const uint32_t selX = st.ix < 0.0f ? kPlaneHi : kPlaneLo, selY = st.iy < 0.0f ? kPlaneHi : kPlaneLo,
+                 selZ = st.iz < 0.0f ? kPlaneHi : kPlaneLo;
+  // A hit child's key is its entry distance with the three lowest bits replaced
+  // by the slot (rounded down, ties in slot order); misses are all ones.
+  uint32_t misses = 0;  // bit k: slot k is missed
+  uint32_t keys[kWideArity];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const float nx = __builtin_fmaf(byte_f(nearX, k), Ax, bnx);
-    const float ny = __builtin_fmaf(byte_f(nearY, k), Ay, bny);
-    const float nz = __builtin_fmaf(byte_f(nearZ, k), Az, bnz);
-    const float fx = __builtin_fmaf(byte_f(farX, k), Ax, bfx);
-    const float fy = __builtin_fmaf(byte_f(farY, k), Ay, bfy);
-    const float fz = __builtin_fmaf(byte_f(farZ, k), Az, bfz);
-    const float tnear = fmaxf(fmaxf(nx, ny), fmaxf(nz, 0.0f));
-    const float tfar = fminf(fminf(fx, fy), fz) * 1.00000095f;
-    tn[k] = ((k < nchild) && tnear <= tfar && tnear <= tbScaled) ? tnear : INFINITY;
+  for (int pair = kWideArity / 2 - 1; pair >= 0; --pair) {
+    const uint32_t next = pair & 1 ? kPlaneNextPair : 0u;
+    const bool high = pair >= 2;  // the words of slots 4..7
+    const uint32_t nx = plane_pair(high ? q2.y : q2.x, high ? q3.w : q3.z, selX ^ next);
+    const uint32_t ny = plane_pair(high ? q2.w : q2.z, high ? q4.y : q4.x, selY ^ next);
+    const uint32_t nz = plane_pair(high ? q3.y : q3.x, high ? q4.w : q4.z, selZ ^ next);
+    const uint32_t fx = plane_pair(high ? q2.y : q2.x, high ? q3.w : q3.z, selX ^ next ^ kPlaneOther);
+    const uint32_t fy = plane_pair(high ? q2.w : q2.z, high ? q4.y : q4.x, selY ^ next ^ kPlaneOther);
+    const uint32_t fz = plane_pair(high ? q3.y : q3.x, high ? q4.w : q4.z, selZ ^ next ^ kPlaneOther);
+#pragma unroll
+    for (int h = 1; h >= 0; --h) {
+      const int k = 2 * pair + h;
+      const float tnear = fmaxf(fmaxf(fmaxf(plane_fma(nx, h, Ax24, bnx), plane_fma(ny, h, Ay24, bny)),
+                                      plane_fma(nz, h, Az24, bnz)), 0.0f);
+      const float tfar = fminf(fminf(fminf(plane_fma(fx, h, Ax24, bfx), plane_fma(fy, h, Ay24, bfy)),
+                                     plane_fma(fz, h, Az24, bfz)), tbScaled);
+      if (ANY) {
+        misses = __builtin_amdgcn_alignbit(misses, __float_as_uint(tfar - tnear), 31);
+      } else {
+        keys[k] = tnear <= tfar ? (__float_as_uint(tnear) & ~7u) | (uint32_t)k : 0xffffffffu;
+        misses = __builtin_amdgcn_alignbit(misses, keys[k], 31);
+      }
+    }
   }
-  float t0 = tn[0], t1 = tn[1], t2 = tn[2], t3 = tn[3];
-  uint32_t c0 = q1.x, c1 = q1.y, c2 = q1.z, c3 = q1.w;
-  if (!ANY) {  // nearest first; missed children (INFINITY) sink to the end
-#define GPUGI_CSWAP(ta, ca, tb_, cb)                       \
-  {                                                        \
-    const bool sw = tb_ < ta;                              \
-    const float lo = sw ? tb_ : ta, hi = sw ? ta : tb_;    \
-    const uint32_t cl = sw ? cb : ca, ch = sw ? ca : cb;   \
-    ta = lo;                                               \
-    tb_ = hi;                                              \
-    ca = cl;                                               \
-    cb = ch;                                               \
+  uint32_t first = 0xffffffffu;  // the smallest key
+  if (!ANY) {
+#pragma unroll
+    for (int k = 0; k < kWideArity; ++k) first = min(first, keys[k]);
   }
-    GPUGI_CSWAP(t0, c0, t1, c1);
-    GPUGI_CSWAP(t2, c2, t3, c3);
-    GPUGI_CSWAP(t0, c0, t2, c2);
-    GPUGI_CSWAP(t1, c1, t3, c3);
-    GPUGI_CSWAP(t1, c1, t2, c2);
-#undef GPUGI_CSWAP
+  const uint32_t inner = q0.w >> 24, hits = ~misses & 0xffu;
+  const uint32_t leaves = hits & ~inner;
+  uint32_t waiting = hits & inner;
+  bool fits = true;
+  st.node = kWideNoNode;
+  if (waiting != 0u) {
+    const uint32_t next = wide_next<ANY>(waiting, first & 7u);
+    st.node = wide_child(q1.x, inner, next);
+    waiting &= ~(1u << next);
+    if (waiting != 0u) {
+      uint32_t e = waiting | (inner << 8);
+      if (!ANY) {
+        // the second smallest key: a distance, since two children or more are hit, and
+        // no larger than those of the children that wait
+        uint32_t a = keys[0], second = 0xffffffffu;
+#pragma unroll
+        for (int k = 1; k < kWideArity; ++k) {
+          second = min(second, max(a, keys[k]));
+          a = min(a, keys[k]);
+        }
+        e |= ((second & 7u) << 16) | (second & kWideBoundMask);
+      }
+      fits = wide_push<B, S>(s, st, stk, make_uint2(q1.x, e));
+    }
   }
-  // The nearest hit inner child is visited next, the nearest hit leaves fill the
-  // free pending slots, every other hit child is pushed (p_k).  Ranks count the
-  // hit inner and hit leaf children nearer than child k; the claims are selects.
-  const float tk[4] = {t0, t1, t2, t3};
-  const uint32_t ck[4] = {c0, c1, c2, c3};
-  int used = 0;
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) used += st.leaf[j] != 0u ? 1 : 0;
-  const int freeSlots = kWidePending - used;
-  uint32_t node = kWideNoNode;
-  uint32_t claimed[kWidePending];
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) claimed[j] = 0u;
-  int nInner = 0, nLeaf = 0;
-  bool pk[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const bool hit = tk[k] != INFINITY;
-    const bool isLeaf = (int32_t)ck[k] < 0;
-    const bool takeNode = hit && !isLeaf && nInner == 0;
-    const bool takeLeaf = hit && isLeaf && nLeaf < freeSlots;
-    node = takeNode ? ck[k] : node;
-#pragma unroll
-    for (int j = 0; j < kWidePending; ++j) claimed[j] = (takeLeaf && nLeaf == j) ? ck[k] : claimed[j];
-    nInner += (hit && !isLeaf) ? 1 : 0;
-    nLeaf += (hit && isLeaf) ? 1 : 0;
-    pk[k] = hit && !takeNode && !takeLeaf;
-  }
-  // free slot j (j >= used) takes claimed[j - used]
-  uint32_t leaf[kWidePending];
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) {
-    uint32_t w = st.leaf[j];
-#pragma unroll
-    for (int u = 0; u <= j; ++u) w = (used == u) ? claimed[j - u] : w;
-    leaf[j] = w;
-  }
-  const bool p0 = pk[0], p1 = pk[1], p2 = pk[2], p3 = pk[3];
-  bool overflow = false;
-  int sp = st.sp;
-  if (sp + 4 <= S) {  // every push stays in LDS: one store and one increment each
-    LdsEntry* e = stk.lds + sp * B + stk.tid;
-    int pushed = 0;
-    if (p3) { e[pushed * B] = make_uint2(c3, __float_as_uint(t3)); ++pushed; }
-    if (p2) { e[pushed * B] = make_uint2(c2, __float_as_uint(t2)); ++pushed; }
-    if (p1) { e[pushed * B] = make_uint2(c1, __float_as_uint(t1)); ++pushed; }
-    if (p0) { e[pushed * B] = make_uint2(c0, __float_as_uint(t0)); ++pushed; }
-    sp += pushed;
-  } else {
-#define GPUGI_PUSH(nd, tv)                                                                  \
-  do {                                                                                      \
-    if (sp < S) {                                                                           \
-      stk.lds[sp * B + stk.tid] = make_uint2((nd), __float_as_uint(tv));                    \
-      ++sp;                                                                                 \
-    } else if ((uint32_t)(sp - S) < s.spillDepth) {                                         \
-      stk.spill[(size_t)(sp - S) * stk.spillStride] = make_uint2((nd), __float_as_uint(tv)); \
-      ++sp;                                                                                 \
-    } else {                                                                                \
-      overflow = true;                                                                      \
-    }                                                                                       \
-  } while (0)
-    if (p3) GPUGI_PUSH(c3, t3);
-    if (p2) GPUGI_PUSH(c2, t2);
-    if (p1) GPUGI_PUSH(c1, t1);
-    if (p0) GPUGI_PUSH(c0, t0);
-#undef GPUGI_PUSH
-  }
-  st.node = node;
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) st.leaf[j] = leaf[j];
-  st.sp = sp;
-  if (overflow) {
+  if (leaves != 0u && !wide_hold(st, nodeIndex, leaves))
+    fits = wide_push<B, S>(s, st, stk, make_uint2(nodeIndex | kWideLeafEntry, leaves | (ANY ? 0u : first & kWideBoundMask))) &&
+           fits;
+  if (!fits) {
     atomicOr(s.errorFlag, 1u);
     st.bestSlot = -2;
-    return false;
   }
-  return true;
+  return fits;
 }
 
-// Leaf pass for a lane with pending leaves: tests their triangles (one loop
-// over the slots in order) and frees every slot.
+// Leaf pass for a lane with pending leaves: tests the triangles of one leaf of
+// the first group.  One leaf a pass: a lane with several does not hold the
+// others' next passes (2^24 diffuse rays on the heightfield: 2460 us with all of
+// a lane's leaves in one pass, 2246 us with one).
 template <bool ANY, bool WT>
 __device__ __forceinline__ void wide_leaf(const WideScene& s, WideState& st) {
   const gg::V3 o = st.o, d = st.d;
-  uint32_t first[kWidePending], end[kWidePending];  // end[j]: triangles of slots 0..j
-  uint32_t cnt = 0;
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) {
-    const uint32_t w = st.leaf[j];
-    first[j] = (w & kWideLeafFirstMask) - cnt;  // triangle of loop index m is first[j] + m
-    cnt += w != 0u ? ((w >> 27) & 0xfu) + 1u : 0u;
-    end[j] = cnt;
-    st.leaf[j] = 0;
-  }
-  for (uint32_t m = 0; m < cnt; ++m) {
-    uint32_t tri = first[kWidePending - 1] + m;
-#pragma unroll
-    for (int j = kWidePending - 2; j >= 0; --j) tri = m < end[j] ? first[j] + m : tri;
+  // {firstChild, firstTri, ends} of the group's node
+  const uint4 q1 = ((const uint4*)((const char*)s.nodes + ((st.leafNode[0] << 6) + (st.leafNode[0] << 4))))[1];
+  const uint32_t shift = 8u * (uint32_t)__builtin_ctz(st.leafMask);
+  uint32_t mask = st.leafMask & (st.leafMask - 1u);
+  const bool last = (mask & 0xffu) == 0u;  // the second group moves up
+  st.leafNode[0] = last ? st.leafNode[1] : st.leafNode[0];
+  st.leafMask = last ? mask >> 8 : mask;
+  const uint64_t ends = (uint64_t)q1.z | ((uint64_t)q1.w << 32);
+  uint32_t tri = q1.y + ((uint32_t)((ends << 8) >> shift) & 0xffu);
+  // empty for an unused slot whose inverted box the slack let through
+  const uint32_t end = q1.y + ((uint32_t)(ends >> shift) & 0xffu);
+  for (; tri < end; ++tri) {
     const size_t ti = 3 * (size_t)tri;
     const float4 a = s.tris[ti + 0];
     const float4 b = s.tris[ti + 1];
@@ -321,58 +343,42 @@ __device__ __forceinline__ void wide_leaf(const WideScene& s, WideState& st) {
 }
 
 // For a lane without a next node: pops entries still in front of the closest
-// hit until one yields a node, or a leaf finds both pending slots taken (the
-// entry stays), or the stack is empty.
-template <int B, int S>
+// hit until one yields a node, or a leaf group finds both pending slots taken
+// (the entry stays), or the stack is empty.
+template <bool ANY, int B, int S>
 __device__ __forceinline__ void wide_pop(WideState& st, const WideStack& stk) {
   const float tb = st.tbest * 1.00000095f;  // entry distances are lower bounds with this slack
   int sp = st.sp;
-  uint32_t leaf[kWidePending];
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) leaf[j] = st.leaf[j];
   uint32_t node = kWideNoNode;
   while (sp > 0) {
     const int top = sp - 1;
-    uint32_t nd;
-    float t;
-    if (top < S) {
-      const uint2 e = stk.lds[top * B + stk.tid];
-      nd = e.x;
-      t = __uint_as_float(e.y);
-    } else {
-      const uint2 e = stk.spill[(size_t)(top - S) * stk.spillStride];
-      nd = e.x;
-      t = __uint_as_float(e.y);
-    }
-    if (t > tb) {
+    uint2 e;
+    if (top < S) e = stk.lds[top * B + stk.tid];
+    else e = stk.spill[(size_t)(top - S) * stk.spillStride];
+    if (!ANY && __uint_as_float(e.y & kWideBoundMask) > tb) {
       sp = top;
       continue;
     }
-    if (nd & kWideLeafFlag) {
-      if (leaf[kWidePending - 1] != 0u) break;
-      bool placed = false;
-#pragma unroll
-      for (int j = 0; j < kWidePending; ++j) {
-        const bool take = !placed && leaf[j] == 0u;
-        leaf[j] = take ? nd : leaf[j];
-        placed = placed || take;
-      }
+    if (e.x & kWideLeafEntry) {
+      if (!wide_hold(st, e.x & ~kWideLeafEntry, e.y & 0xffu)) break;
       sp = top;
       continue;
     }
-    node = nd;
-    sp = top;
+    const uint32_t next = wide_next<ANY>(e.y & 0xffu, (e.y >> 16) & 7u);  // a node entry has a waiting child
+    node = wide_child(e.x, (e.y >> 8) & 0xffu, next);
+    e.y &= ~(1u << next);
+    if ((e.y & 0xffu) == 0u) sp = top;
+    else if (top < S) stk.lds[top * B + stk.tid].y = e.y;
+    else stk.spill[(size_t)(top - S) * stk.spillStride].y = e.y;
     break;
   }
   st.sp = sp;
-#pragma unroll
-  for (int j = 0; j < kWidePending; ++j) st.leaf[j] = leaf[j];
   st.node = node;
 }
 
 // Wave-uniform pass choice for the working lanes (mask `working`, a ballot
 // taken by the caller): a leaf pass when no working lane has a node to visit
-// or at least `waitLanes` of them have only a pending leaf.
+// or at least `waitLanes` of them have only pending leaves.
 __device__ __forceinline__ bool wide_choose_leaf_pass(uint64_t working, const WideState& st, int waitLanes) {
   const uint64_t hasNode = __ballot(st.node != kWideNoNode);
   return (working & hasNode) == 0 || __popcll(working & ~hasNode) >= waitLanes;
@@ -382,7 +388,7 @@ __device__ __forceinline__ bool wide_choose_leaf_pass(uint64_t working, const Wi
 template <bool ANY, int B, int S, bool WT>
 __device__ __forceinline__ bool wide_pass(const WideScene& s, WideState& st, bool leafPass, const WideStack& stk) {
   if (leafPass) {
-    if (st.leaf[0] == 0u) return false;  // still traversing; unaffected by this pass
+    if (st.leafMask == 0u) return false;  // still traversing; unaffected by this pass
     wide_leaf<ANY, WT>(s, st);
     if (ANY && st.found) return true;
   } else {
@@ -390,8 +396,8 @@ __device__ __forceinline__ bool wide_pass(const WideScene& s, WideState& st, boo
     if (!wide_visit<ANY, B, S>(s, st, stk)) return true;  // overflow, slot -2
   }
   if (st.node == kWideNoNode) {
-    wide_pop<B, S>(st, stk);
-    return st.node == kWideNoNode && st.leaf[0] == 0u;
+    wide_pop<ANY, B, S>(st, stk);
+    return st.node == kWideNoNode && st.leafMask == 0u;
   }
   return false;
 }
@@ -409,7 +415,8 @@ __device__ __forceinline__ WideResult trace_wide_ray(const WideScene& s, gg::V3 
   for (;;) {
     const uint64_t act = __ballot(live);
     if (act == 0) break;
-    const bool leafPass = wide_choose_leaf_pass(act, st, (__popcll(act) + 1) / 2);
+    // a quarter of the live lanes: 3 % (room, path tracer) below a half; an eighth is the same
+    const bool leafPass = wide_choose_leaf_pass(act, st, (__popcll(act) + 3) / 4);
     if (live && wide_pass<ANY, B, S, WT>(s, st, leafPass, stk)) live = false;
   }
   WideResult r;

@@ -1,4 +1,4 @@
-// Persistent-wave ray queries on the 4-wide quantized BVH.
+// Persistent-wave ray queries on the 8-wide quantized BVH.
 //
 // Scheduling: workgroups are dispatched round-robin over the 8 XCDs, so block
 // b runs on XCD b % 8; XCD x owns the x-th contiguous eighth of the ray array
@@ -14,6 +14,16 @@
 // refill = 64 reproduces batch-at-a-time processing.
 // The LDS stack depth is a template parameter: deeper stacks spill less but
 // cap the waves per CU (160 KiB LDS per CU); the autotuner picks it.
+//
+// Bound by VALU issue (1.13 wave-instructions per CU and cycle, an FMA stream
+// reaches 0.99) and by the vector-memory data path (TD busy 94 % of the cycles)
+// at once, so a node holds eight children in five 16-byte loads: against
+// four-child nodes of four loads, 0.67 times the node visits and about the
+// same instructions per visit.  Measured (2^24 diffuse rays, 2,097,152-triangle
+// heightfield; 2^22 camera / diffuse / shadow rays, 5,120,016-triangle room):
+// four children 2471 us; 3054 / 1889 / 1193 us; eight 2194; 1526 / 1413 / 953 us.
+// Seven waves per SIMD (72 VGPRs, no spill): six measured 2282 us on the
+// heightfield set, eight spill 44 bytes a lane in the box pass and take 3248 us.
 // Compiled with -ffp-contract=off: the triangle test must round exactly like
 // the reference formula.
 #include <hip/hip_runtime.h>
@@ -30,7 +40,7 @@ __global__ void k_wide_queue_reset(uint32_t* q) {
 }
 
 template <bool ANY, int B, int S, bool WT>
-__global__ __launch_bounds__(B) void k_trace_wide(WideScene s, const float4* __restrict__ rays,
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_trace_wide(WideScene s, const float4* __restrict__ rays,
                                                   int4* __restrict__ hits, uint32_t n, int refill, int wait,
                                                   const uint32_t* __restrict__ nDev) {
   __shared__ uint2 lds[S * B];

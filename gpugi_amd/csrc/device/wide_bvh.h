@@ -1,11 +1,18 @@
-// Re-packed 4-wide BVH with 8-bit quantized child boxes (host layout + device view).
+// Re-packed 8-wide BVH with 8-bit quantized child boxes (host layout + device view).
 //
-// Node: 64 bytes, read as four 16-byte loads (one half of a 128-byte L2 line):
-//   q0 = {origin.x, origin.y, origin.z, exps}   exps = ex | ey<<8 | ez<<16 | nchild<<24,
+// Node: 80 bytes, read as five 16-byte loads:
+//   q0 = {origin.x, origin.y, origin.z, exps}   exps = ex | ey<<8 | ez<<16 | inner<<24,
 //                                              scale_a = 2^(e_a - 127)
-//   q1 = {child[0..3]}                          inner: node index; leaf: MSB | (count-1)<<27 | first
-//   q2 = {lo.x[4], lo.y[4], lo.z[4], hi.x[4]}   one byte per child
-//   q3 = {hi.y[4], hi.z[4], 0, 0}
+//   q1 = {firstChild, firstTri, ends[0..7]}     ends: one byte per child
+//   q2 = {lo.x[8], lo.y[8]}, q3 = {lo.z[8], hi.x[8]}, q4 = {hi.y[8], hi.z[8]}
+// A child sits in one of eight slots.  Bit k of `inner` marks slot k as an inner
+// node; the inner children are consecutive nodes from firstChild in slot order.
+// Any other slot is a leaf whose triangles are firstTri + [ends[k-1], ends[k])
+// (ends[-1] = 0), which is empty for an unused slot; an unused slot also has
+// the inverted box lo = 255, hi = 0.  Slots are in the order of the child boxes'
+// surface, smallest first.  (Compressed eight-wide nodes: Ylitie, Karras and
+// Laine 2017, "Efficient incoherent ray traversal on GPUs through compressed
+// wide BVHs".)
 // child box along axis a = [origin_a + lo*scale_a, origin_a + hi*scale_a]; the
 // host rounds lo down and hi up and checks in extended precision that the
 // exact origin + q * scale encloses the child box, so the quantized tree is conservative.
@@ -26,19 +33,21 @@
 
 namespace gpugi {
 
-constexpr uint32_t kWideLeafFlag = 0x80000000u;
-constexpr uint32_t kWideLeafFirstMask = (1u << 27) - 1;
-constexpr uint32_t kWideMaxLeafTris = 16;
+constexpr int kWideArity = 8;
+constexpr uint32_t kWideNodeBytes = 80;
+constexpr uint32_t kWideMaxTris = 1u << 27;
+constexpr uint32_t kWideMaxNodes = 1u << 25;  // node offsets stay below 2^32 bytes
+constexpr uint32_t kWideMaxLeafTris = 16;     // ends[7] <= 8 * 16 fits its byte
 
 struct WideNodeHost {
   float origin[3];
   uint32_t exps;
-  uint32_t child[4];
-  uint8_t lo[3][4];
-  uint8_t hi[3][4];
-  uint32_t pad[2];
+  uint32_t firstChild, firstTri;
+  uint8_t ends[kWideArity];
+  uint8_t lo[3][kWideArity];
+  uint8_t hi[3][kWideArity];
 };
-static_assert(sizeof(WideNodeHost) == 64, "wide node is 64 bytes");
+static_assert(sizeof(WideNodeHost) == kWideNodeBytes, "wide node is 80 bytes");
 
 struct WideTriHost {
   float p0[3];
@@ -53,12 +62,13 @@ static_assert(sizeof(WideTriHost) == 48, "wide triangle is 48 bytes");
 struct WideBVHHost {
   std::vector<WideNodeHost> nodes;
   std::vector<WideTriHost> tris;
-  uint32_t maxStack = 0;   // worst-case traversal stack entries (siblings summed along a path)
+  uint32_t maxPending = 0;  // most children that can wait on a traversal stack (siblings summed along a path)
+  uint32_t maxStack = 0;    // most stack entries those take (an entry holds the waiting children of one node)
   uint32_t depth = 0;
 };
 
-// Re-packs the reference BVH2 (any arity written in preorder with escape
-// pointers) into the 4-wide quantized layout.  Leaves of up to
+// Re-packs the reference BVH2 (any arity up to 8 written in preorder with escape
+// pointers) into the 8-wide quantized layout.  Leaves of up to
 // `maxLeafTris` triangles are formed from subtrees that small.  rawVertices:
 // triangles store {p0, slot}{p1, mat}{p2, 0} (watertight test) instead of the
 // reference test's operands {p0, slot}{p1 - p0, mat}{p0 - p2, 0}.
@@ -71,7 +81,7 @@ constexpr int kWideLdsStack = 16;
 
 #if defined(__HIPCC__)
 struct WideScene {
-  const uint4* __restrict__ nodes;    // 4 x uint4 per node
+  const uint4* __restrict__ nodes;    // 5 x uint4 per node
   const float4* __restrict__ tris;    // 3 x float4 per triangle
   uint2* spill;                       // per-thread overflow stack (global memory)
   uint32_t spillDepth;                // entries per thread in `spill`

@@ -1,4 +1,4 @@
-// Re-pack of the reference BVH2 into the 4-wide quantized layout of wide_bvh.h.
+// Re-pack of the reference BVH2 into the 8-wide quantized layout of wide_bvh.h.
 #include "../device/wide_bvh.h"
 
 #include <algorithm>
@@ -24,24 +24,6 @@ struct Bvh2View {
   }
 };
 
-// Children of an inner node: firstChild, then escapes until the chain leaves
-// the parent (the last child escapes to the parent's escape).
-bool Children(const Bvh2View& v, uint32_t i, std::vector<uint32_t>* out, std::string* err) {
-  out->clear();
-  uint32_t c = v.firstChild(i);
-  const uint32_t stop = v.escape(i);
-  for (int guard = 0; guard < 64; ++guard) {
-    if (c <= i || c >= v.n) { *err = "malformed hierarchy below node " + std::to_string(i); return false; }
-    out->push_back(c);
-    uint32_t e = v.escape(c);
-    if (e == stop) return true;
-    if (e <= c) { *err = "malformed escape chain below node " + std::to_string(i); return false; }
-    c = e;
-  }
-  *err = "node " + std::to_string(i) + " has more than 64 children";
-  return false;
-}
-
 // The exact real origin + q * scale (extended precision: the kernel never rounds a
 // decoded bound, it folds q * scale into the slab distance).
 long double Decode(float origin, uint32_t q, float scale) {
@@ -52,46 +34,60 @@ float ScaleOf(uint32_t biased) { uint32_t u = biased << 23; float f; std::memcpy
 }  // namespace
 
 std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, WideBVHHost* out, bool rawVertices) {
+  constexpr int W = kWideArity;
   if (maxLeafTris < 1 || maxLeafTris > kWideMaxLeafTris) return "maxLeafTris must be in [1, 16]";
   Bvh2View v{&desc, desc.num_nodes};
   if (v.n == 0) return "empty hierarchy";
   const uint32_t tpl = desc.triangles_per_leaf;
-  std::string err;
+  // Children of every inner node: firstChild, then escapes until the chain leaves
+  // the parent (the last child escapes to the parent's escape); node i's are
+  // kids[kidsAt[i]..kidsAt[i + 1]).
+  std::vector<uint32_t> kids, kidsAt(v.n + 1, 0);
+  kids.reserve(v.n);
+  for (uint32_t i = 0; i < v.n; ++i) {
+    kidsAt[i] = (uint32_t)kids.size();
+    if (v.isLeafNode(i)) continue;
+    uint32_t c = v.firstChild(i);
+    const uint32_t stop = v.escape(i);
+    for (int guard = 0;; ++guard) {
+      if (guard == 64) return "node " + std::to_string(i) + " has more than 64 children";
+      if (c <= i || c >= v.n) return "malformed hierarchy below node " + std::to_string(i);
+      kids.push_back(c);
+      const uint32_t e = v.escape(c);
+      if (e == stop) break;
+      if (e <= c) return "malformed escape chain below node " + std::to_string(i);
+      c = e;
+    }
+  }
+  kidsAt[v.n] = (uint32_t)kids.size();
   // Subtree valid-triangle counts, bottom-up (children follow parents in preorder).
   std::vector<uint32_t> count(v.n, 0);
-  std::vector<std::vector<uint32_t>> kids(v.n);
-  for (uint32_t i = 0; i < v.n; ++i) {
-    if (v.isLeafNode(i)) continue;
-    if (!Children(v, i, &kids[i], &err)) return err;
-  }
   for (uint32_t ii = v.n; ii-- > 0;) {
+    uint32_t c = 0;
     if (v.isLeafNode(ii)) {
       uint32_t leaf = v.firstChild(ii) & 0x7fffffffu;
       if (leaf >= desc.num_leaves) return "leaf index out of range";
-      uint32_t c = 0;
       for (uint32_t k = 0; k < tpl; ++k) {
         const int32_t* t = desc.triangles + ((size_t)leaf * tpl + k) * 4;
         if (t[0] == t[1]) break;
         ++c;
       }
-      count[ii] = c;
     } else {
-      uint32_t c = 0;
-      for (uint32_t k : kids[ii]) c += count[k];
-      count[ii] = c;
+      for (uint32_t k = kidsAt[ii]; k < kidsAt[ii + 1]; ++k) c += count[kids[k]];
     }
+    count[ii] = c;
   }
   out->nodes.clear();
   out->tris.clear();
   out->tris.reserve(count[0]);
 
-  auto appendTris = [&](uint32_t sub) -> uint32_t {
+  std::vector<uint32_t> walk;
+  auto appendTris = [&](uint32_t sub) {
     // All valid slots of a BVH2 subtree in slot order of a preorder walk.
-    uint32_t first = (uint32_t)out->tris.size();
-    std::vector<uint32_t> st{sub};
-    while (!st.empty()) {
-      uint32_t i = st.back();
-      st.pop_back();
+    walk.assign(1, sub);
+    while (!walk.empty()) {
+      uint32_t i = walk.back();
+      walk.pop_back();
       if (v.isLeafNode(i)) {
         uint32_t leaf = v.firstChild(i) & 0x7fffffffu;
         for (uint32_t k = 0; k < tpl; ++k) {
@@ -114,113 +110,99 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
           out->tris.push_back(w);
         }
       } else {
-        for (size_t k = kids[i].size(); k-- > 0;) st.push_back(kids[i][k]);
+        for (uint32_t k = kidsAt[i + 1]; k-- > kidsAt[i];) walk.push_back(kids[k]);
       }
     }
-    return first;
   };
 
-  // SAH-optimal collapse of the BVH2 into 4-wide nodes (the dynamic program of
-  // Ylitie, Karras and Laine 2017, "Efficient incoherent ray traversal on
-  // GPUs through compressed wide BVHs").  dist[n][j] is the least expected
-  // cost of covering n's subtree with at most j children of one wide node;
-  // a child is a leaf (a reference leaf, or a subtree of at most maxLeafTris
-  // valid triangles) or a wide node of its own.  A wide node costs
-  // kNodeCost * area per visit, a leaf kTriCost * area * triangles; the ratio
-  // is the measured cost of a box pass (four slab tests, ordering, stack) to
-  // that of one triangle test.  The topology stays the reference's: only which
-  // BVH2 nodes become wide nodes or leaves is chosen.
+  // SAH-optimal collapse of the BVH2 into 8-wide nodes (the dynamic program of
+  // Ylitie, Karras and Laine 2017).  dist[n][j] is the least expected cost of
+  // covering n's subtree with at most j children of one wide node; a child is a
+  // leaf (a reference leaf, or a subtree of at most maxLeafTris valid triangles)
+  // or a wide node of its own.  A wide node costs kNodeCost * area per visit, a
+  // leaf kTriCost * area * triangles; the ratio is the measured cost of a box
+  // pass (the slab tests, ordering, stack) to that of one triangle test.  The
+  // topology stays the reference's: only which BVH2 nodes become wide nodes or
+  // leaves is chosen.
   constexpr float kNodeCost = 1.0f, kTriCost = 0.4f;
   constexpr float kInf = std::numeric_limits<float>::infinity();
   struct Dp {
-    float dist[5];
-    uint8_t pick[5];     // 0: no child (empty subtree), 1: n as one child, 2: n's children share j
-    bool leaf;           // n as one child: a leaf (else a wide node)
+    float dist[W + 1];
+    uint8_t pick[W + 1];  // 0: no child (empty subtree), 1: n as one child, 2: n's children share j
+    bool leaf;            // n as one child: a leaf (else a wide node)
+    bool open;            // n's own children fit one wide node
   };
   std::vector<Dp> dp(v.n);
-  // split[splitAt[i] + k][j]: children given to kid k when kids 0..k of node i
+  // split[kidsAt[i] + k][j]: children given to kid k when kids 0..k of node i
   // share j (knapsack back-pointers)
-  std::vector<size_t> splitAt(v.n + 1, 0);
-  for (uint32_t i = 0; i < v.n; ++i) splitAt[i + 1] = splitAt[i] + kids[i].size();
-  std::vector<std::array<uint8_t, 5>> split(splitAt[v.n], std::array<uint8_t, 5>{0, 0, 0, 0, 0});
+  typedef std::array<uint8_t, W + 1> Split;
+  std::vector<Split> split(kids.size(), Split{});
   for (uint32_t n = v.n; n-- > 0;) {
     Dp& d = dp[n];
     if (count[n] == 0) {
-      for (int j = 0; j < 5; ++j) { d.dist[j] = 0.0f; d.pick[j] = 0; }
-      d.leaf = true;
+      for (int j = 0; j <= W; ++j) { d.dist[j] = 0.0f; d.pick[j] = 0; }
+      d.leaf = d.open = true;
       continue;
     }
     const float area = v.surface(n);
     const bool leafOk = v.isLeafNode(n) || count[n] <= maxLeafTris;
     const float leafCost = leafOk ? kTriCost * area * (float)count[n] : kInf;
-    std::array<float, 5> comb = {0.0f, kInf, kInf, kInf, kInf};
+    std::array<float, W + 1> comb;
+    comb.fill(kInf);
     if (!v.isLeafNode(n)) {
-      for (size_t k = 0; k < kids[n].size(); ++k) {
-        const Dp& c = dp[kids[n][k]];
-        std::array<float, 5> next = {kInf, kInf, kInf, kInf, kInf};
-        for (int j = 0; j < 5; ++j)
+      comb[0] = 0.0f;
+      for (uint32_t k = kidsAt[n]; k < kidsAt[n + 1]; ++k) {
+        const Dp& c = dp[kids[k]];
+        std::array<float, W + 1> next;
+        next.fill(kInf);
+        for (int j = 0; j <= W; ++j)
           for (int a = 0; a <= j; ++a) {
             const float cost = comb[j - a] + c.dist[a];
-            if (cost < next[j]) { next[j] = cost; split[splitAt[n] + k][j] = (uint8_t)a; }
+            if (cost < next[j]) { next[j] = cost; split[k][j] = (uint8_t)a; }
           }
         comb = next;
       }
-    } else {
-      comb = {kInf, kInf, kInf, kInf, kInf};
     }
-    const float nodeCost = v.isLeafNode(n) ? kInf : kNodeCost * area + comb[4];
+    const float nodeCost = v.isLeafNode(n) ? kInf : kNodeCost * area + comb[W];
     const float single = std::min(leafCost, nodeCost);
     d.leaf = leafCost <= nodeCost;
+    d.open = v.isLeafNode(n) || comb[W] < kInf;
     d.dist[0] = kInf;
     d.pick[0] = 0;
-    for (int j = 1; j < 5; ++j) {
+    for (int j = 1; j <= W; ++j) {
       if (single <= comb[j]) { d.dist[j] = single; d.pick[j] = 1; }
       else { d.dist[j] = comb[j]; d.pick[j] = 2; }
     }
   }
-  // The children of the wide node for BVH2 node n: n's own children sharing 4.
+  // The children of the wide node for BVH2 node n: n's own children sharing W.
   struct Item {
     uint32_t bvh2;
     bool leaf;
   };
   std::vector<Item> items;
-  std::vector<std::pair<uint32_t, int>> work;  // (node, children it may use)
+  std::vector<std::pair<uint32_t, int>> work;  // (BVH2 node, children it may use), last first
+  auto openKids = [&](uint32_t n, int j) {  // knapsack back-tracking over n's kids
+    for (uint32_t k = kidsAt[n + 1]; k-- > kidsAt[n];) {
+      const int a = split[k][j];
+      work.push_back({kids[k], a});
+      j -= a;
+    }
+  };
   auto wideChildren = [&](uint32_t n) {
     items.clear();
     if (v.isLeafNode(n)) {  // a one-leaf scene
       if (count[n] > 0) items.push_back({n, true});
       return;
     }
-    // knapsack back-tracking over n's kids, then each kid's own choice
     work.clear();
-    int j = 4;
-    std::vector<std::pair<uint32_t, int>> alloc;
-    for (size_t k = kids[n].size(); k-- > 0;) {
-      const int a = split[splitAt[n] + k][j];
-      alloc.push_back({kids[n][k], a});
-      j -= a;
-    }
-    for (size_t k = alloc.size(); k-- > 0;) work.push_back(alloc[k]);
-    // expand in child order
-    for (size_t w = 0; w < work.size(); ++w) {
-      const uint32_t c = work[w].first;
-      const int jc = work[w].second;
+    openKids(n, W);
+    while (!work.empty()) {  // in the reference's child order
+      const auto [c, j] = work.back();
+      work.pop_back();
       const Dp& d = dp[c];
-      if (jc == 0 || d.pick[jc] == 0) continue;
-      if (d.pick[jc] == 1) {
-        items.push_back({c, d.leaf});
-        continue;
-      }
-      // c opened: its kids share jc, inserted in place to keep the reference's child order
-      std::vector<std::pair<uint32_t, int>> sub;
-      int jj = jc;
-      for (size_t k = kids[c].size(); k-- > 0;) {
-        const int a = split[splitAt[c] + k][jj];
-        sub.push_back({kids[c][k], a});
-        jj -= a;
-      }
-      std::reverse(sub.begin(), sub.end());
-      work.insert(work.begin() + (std::ptrdiff_t)w + 1, sub.begin(), sub.end());
+      if (j == 0 || d.pick[j] == 0) continue;
+      if (d.pick[j] == 1) items.push_back({c, d.leaf});
+      else openKids(c, j);
     }
   };
 
@@ -231,25 +213,23 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
   std::vector<Pending> todo;
   out->nodes.push_back(WideNodeHost());
   todo.push_back({0, 0});
-  std::vector<uint32_t> needStack;   // per wide node: worst-case stack entries below it
-  std::vector<std::vector<uint32_t>> wideKids;
-  needStack.push_back(0);
-  wideKids.emplace_back();
   while (!todo.empty()) {
     Pending p = todo.back();
     todo.pop_back();
     // Subtrees without a valid triangle never produce a hit and are left out.
     wideChildren(p.bvh2);
-    if (items.size() > 4) return "BVH node with more than 4 children cannot be packed";
-    if (items.empty()) {  // a scene without any valid triangle
-      WideNodeHost empty;
-      std::memset(&empty, 0, sizeof(empty));
-      empty.exps = 1u | (1u << 8) | (1u << 16);
-      out->nodes[p.wideIndex] = empty;
-      continue;
-    }
+    std::stable_sort(items.begin(), items.end(),
+                     [&](const Item& a, const Item& b) { return v.surface(a.bvh2) < v.surface(b.bvh2); });
+    if (!dp[p.bvh2].open) return "BVH node with more than 8 children cannot be packed";
     WideNodeHost node;
     std::memset(&node, 0, sizeof(node));
+    std::memset(node.lo, 255, sizeof(node.lo));  // unused slots: inverted boxes, no triangles
+    node.firstTri = (uint32_t)out->tris.size();
+    if (items.empty()) {  // a scene without any valid triangle
+      node.exps = 1u | (1u << 8) | (1u << 16);
+      out->nodes[p.wideIndex] = node;
+      continue;
+    }
     // Quantization frame.
     float origin[3], top[3];
     for (int a = 0; a < 3; ++a) {
@@ -287,48 +267,47 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
       }
       biased[a] = (uint32_t)b;
     }
-    node.exps = biased[0] | (biased[1] << 8) | (biased[2] << 16) | ((uint32_t)items.size() << 24);
-    uint32_t innerKids = 0;
-    for (size_t k = 0; k < items.size(); ++k) {
-      const uint32_t it = items[k].bvh2;
-      if (items[k].leaf) {
-        uint32_t c = count[it];
-        uint32_t first = appendTris(it);
-        if (first > kWideLeafFirstMask) return "too many triangles for the wide layout";
-        node.child[k] = kWideLeafFlag | ((c - 1) << 27) | first;
-      } else {
-        uint32_t wi = (uint32_t)out->nodes.size();
-        out->nodes.push_back(WideNodeHost());
-        needStack.push_back(0);
-        wideKids.emplace_back();
-        wideKids[p.wideIndex].push_back(wi);
-        node.child[k] = wi;
-        todo.push_back({it, wi});
-        ++innerKids;
-      }
+    uint32_t inner = 0, numInner = 0;
+    for (size_t s = 0; s < (size_t)W; ++s) {
+      if (s < items.size() && items[s].leaf) appendTris(items[s].bvh2);
+      else if (s < items.size()) { inner |= 1u << s; ++numInner; }
+      node.ends[s] = (uint8_t)(out->tris.size() - node.firstTri);
     }
-    node.pad[0] = innerKids;  // used for the stack bound only
+    if (out->tris.size() > kWideMaxTris) return "too many triangles for the wide layout";
+    node.firstChild = (uint32_t)out->nodes.size();
+    if (node.firstChild + numInner > kWideMaxNodes) return "too many nodes for the wide layout";
+    out->nodes.resize(out->nodes.size() + numInner);
+    for (int s = W, i = (int)numInner; s-- > 0;)
+      if ((inner >> s) & 1) todo.push_back({items[s].bvh2, node.firstChild + (uint32_t)--i});
+    node.exps = biased[0] | (biased[1] << 8) | (biased[2] << 16) | (inner << 24);
     out->nodes[p.wideIndex] = node;
   }
-  // Worst-case stack.  A visit pushes every hit child except the nearest inner
-  // one, which is visited next (leaf children are pushed when the lane's
-  // pending-leaf slot is taken), so need(n) = (children - [n has an inner
-  // child]) + max need(inner child); popped leaf entries push nothing.  Wide
-  // nodes are numbered parent-before-child, so a reverse sweep is bottom-up.
-  uint32_t depthMax = 1;
-  std::vector<uint32_t> depth(out->nodes.size(), 1);
-  for (size_t i = 0; i < out->nodes.size(); ++i)
-    for (uint32_t c : wideKids[i]) { depth[c] = depth[i] + 1; depthMax = std::max(depthMax, depth[c]); }
+  // Worst-case stack.  A visit goes on with one hit inner child; the other hit
+  // inner children wait in one entry, and the hit leaves in another when both
+  // pending-leaf slots of the lane are taken, so
+  //   stack(n) = [n has two inner children] + [n has a leaf] + max stack(inner child).
+  // An entry that waits keeps its place while children of it are visited, which
+  // the sum covers.  Children are numbered after their parents.
+  std::vector<uint32_t> stack(out->nodes.size(), 0), pending(out->nodes.size(), 0), depth(out->nodes.size(), 1);
   for (size_t i = out->nodes.size(); i-- > 0;) {
-    uint32_t m = 0;
-    for (uint32_t c : wideKids[i]) m = std::max(m, needStack[c]);
-    const uint32_t k = out->nodes[i].pad[0];
-    const uint32_t children = out->nodes[i].exps >> 24;
-    needStack[i] = (k > 0 ? children - 1 : children) + m;
-    out->nodes[i].pad[0] = 0;
+    const WideNodeHost& n = out->nodes[i];
+    const uint32_t numInner = (uint32_t)__builtin_popcount(n.exps >> 24);
+    uint32_t leaves = 0, end = 0;
+    for (int s = 0; s < W; ++s) {
+      leaves += n.ends[s] > end ? 1 : 0;
+      end = n.ends[s];
+    }
+    for (uint32_t c = n.firstChild; c < n.firstChild + numInner; ++c) {
+      stack[i] = std::max(stack[i], stack[c]);
+      pending[i] = std::max(pending[i], pending[c]);
+      depth[i] = std::max(depth[i], depth[c] + 1);
+    }
+    stack[i] += (numInner > 1 ? 1 : 0) + (leaves > 0 ? 1 : 0);
+    pending[i] += numInner + leaves - (numInner > 0 ? 1 : 0);
   }
-  out->maxStack = needStack[0];
-  out->depth = depthMax;
+  out->maxStack = stack[0];
+  out->maxPending = pending[0];
+  out->depth = depth[0];
   return std::string();
 }
 

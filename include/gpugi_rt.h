@@ -49,7 +49,7 @@ enum gpugi_query {
 enum gpugi_kernel {
   GPUGI_KERNEL_AUTO = 0,      /* fastest kernel available for the loaded scene */
   GPUGI_KERNEL_REFERENCE = 1, /* escape-pointer walk on the reference BVH2 layout (bit-exact) */
-  GPUGI_KERNEL_WIDE = 2       /* ordered walk on the re-packed quantized 4-wide BVH */
+  GPUGI_KERNEL_WIDE = 2       /* ordered walk on the re-packed quantized 8-wide BVH */
 };
 
 /* Path schedules of gpugi_set_pt_schedule. */
@@ -187,7 +187,7 @@ int gpugi_set_triangle_test(gpugi_ctx* ctx, int mode);
  * hierarchy (the reference reads them from its scene library, not in the
  * tree; see gpugi_hostscene_obox_hierarchy) and the reference walk
  * (GPUGI_KERNEL_REFERENCE, in gpugi_trace and the integrators) tests those;
- * the wide kernel keeps its own axis-aligned 4-wide tree. */
+ * the wide kernel keeps its own axis-aligned 8-wide tree. */
 int gpugi_set_bvh_type(gpugi_ctx* ctx, int bvh_type);
 /* Bounce from which Russian roulette runs (default 0: every bounce, as
  * pathtracer.comp:99-104 and lighttracer.comp:183-188 do; 3 gives the
@@ -202,7 +202,7 @@ int gpugi_set_rr_start_depth(gpugi_ctx* ctx, int depth);
  * draws fail with GPUGI_ERR_STATE while it is set. */
 int gpugi_set_specific_path_length(gpugi_ctx* ctx, int length);
 /* Traversal the integrators use: GPUGI_KERNEL_REFERENCE (bit-exact escape
- * walk) or GPUGI_KERNEL_WIDE / GPUGI_KERNEL_AUTO (4-wide quantized BVH).
+ * walk) or GPUGI_KERNEL_WIDE / GPUGI_KERNEL_AUTO (8-wide quantized BVH).
  * Replaces the AABOX_BVH define of the shader compile (pathtracer.cpp:55-64). */
 int gpugi_set_integrator_kernel(gpugi_ctx* ctx, int kernel);
 /* How gpugi_draw(GPUGI_PT) schedules the paths, and gpugi_draw(GPUGI_BPT) its
@@ -408,10 +408,12 @@ int gpugi_trace(gpugi_ctx* ctx, int query, int kernel, const gpugi_ray* rays, gp
  * kernel (4, 8, 10, 12, 16 or 24; deeper entries spill to global memory), the
  * number of idle lanes (1..64) at which a wave refills them with new rays and
  * the number of lanes (1..64) waiting with a pending leaf at which a wave runs
- * a triangle pass instead of a box pass.  Default (2, 10, 8, 16): the fastest
+ * a triangle pass instead of a box pass.  Default (2, 10, 8, 8): the fastest
  * incoherent closest-hit configuration on the 2,097,152-triangle heightfield.  No
  * reference counterpart: the GLSL path has one fixed layout
- * (TRIANGLES_PER_LEAF, scenedata.glsl:5). */
+ * (TRIANGLES_PER_LEAF, scenedata.glsl:5).  A stack entry holds the children of
+ * one node that wait; gpugi_get_wide_config's max_stack is the most children
+ * that can wait on one ray's stack in the loaded scene. */
 int gpugi_set_wide_config(gpugi_ctx* ctx, int max_leaf_triangles, int lds_stack_entries, int refill_lanes,
                           int wait_lanes);
 int gpugi_get_wide_config(gpugi_ctx* ctx, int* max_leaf_triangles, int* lds_stack_entries, int* refill_lanes,
@@ -639,7 +641,7 @@ int gpugi_batch_add(gpugi_batch* batch, const gpugi_scene_desc* scene, const gpu
 /* Packs and uploads all scenes; then gpugi_batch_reset(batch, 0). */
 int gpugi_batch_finalize(gpugi_batch* batch);
 /* Traversal (GPUGI_KERNEL_REFERENCE: the BVH2 escape walk, GPUGI_KERNEL_WIDE:
- * the 4-wide BVH), tiles taken per queue access, the persistent grid in
+ * the 8-wide BVH), tiles taken per queue access, the persistent grid in
  * quarters of full residency (1..16) and the wide walk's LDS stack entries
  * per lane (16, 24 or 32; deeper entries spill to global memory; the escape
  * walk ignores it).  Defaults: WIDE, 2, 2, 16. */

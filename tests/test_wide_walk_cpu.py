@@ -1,0 +1,126 @@
+"""The wide BVH re-pack and the wide traversal on the CPU: the device functions
+of trace_wide.h compiled for the host (tests/native/wide_walk_host.cpp) against
+the oracle's brute force over all triangles, every ray record bit for bit.
+
+Both evaluate the same float triangle test and take the nearest hit, the
+smaller slot on a tie, so no tolerance is needed unless a box rejects a hit.
+"""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from gpugi_amd import rt as _rt
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def walk(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("walk") / "wide_walk.so")
+    csrc = os.path.join(ROOT, "gpugi_amd", "csrc")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-w", "-fPIC", "-shared",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + csrc, "-isystem", "/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "native", "wide_walk_host.cpp"),
+                    os.path.join(csrc, "host", "wide_bvh.cpp"), "-o", lib], check=True)
+    fn = ctypes.CDLL(lib).wide_walk
+
+    def run(scene, rays, leaf=2, any_hit=False, watertight=False, lds=10):
+        rays = np.ascontiguousarray(rays, np.float32)
+        hits, counts = np.zeros((len(rays), 4), np.int32), np.zeros(6, np.uint32)
+        p = ctypes.c_void_p
+        assert fn(ctypes.byref(scene.desc()), ctypes.c_uint32(leaf), int(any_hit), int(watertight), lds,
+                  p(rays.ctypes.data), p(hits.ctypes.data), ctypes.c_size_t(len(rays)), p(counts.ctypes.data)) == 0
+        assert counts[5] == 0 and counts[4] <= counts[3]  # no overflow, the stack bound holds
+        return hits, dict(zip(("nodes", "tris", "pending", "stack", "used"), counts.tolist()))
+    return run
+
+
+def ray_set(scene, n, seed):
+    """Rays between random points in and around the scene, a quarter of them along an axis."""
+    rng = np.random.default_rng(seed)
+    info = scene.info()
+    lo, hi = np.array(info["bbox_min"]), np.array(info["bbox_max"])
+    ext = hi - lo
+    o, t = lo + ext * (1.4 * rng.random((n, 3)) - 0.2), lo + ext * rng.random((n, 3))
+    d = t - o
+    axis = rng.integers(0, 3, n // 4)
+    d[:n // 4] = 0.0
+    d[np.arange(n // 4), axis] = rng.choice([-1.0, 1.0], n // 4)
+    d[:n // 8] = -d[:n // 8]  # zeros of either sign
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    r = np.zeros((n, 8), np.float32)
+    r[:, 0:3], r[:, 4:7] = o, d
+    r[:, 3] = np.where(rng.random(n) < 0.5, np.float32(3.402823466e38), np.linalg.norm(ext) * rng.random(n))
+    return r
+
+
+def nested_scene(levels):
+    """Quads around the origin, three per level and each level a third of the last in size: a deep, narrow
+    tree.  (The float triangle test is noise on the smallest ones: only a brute force over all of them, not a
+    walk with its own box test, gives the walk's answers.)"""
+    pos, idx, s = [], [], 1.0
+    for _ in range(levels):
+        for a in range(3):
+            c = np.zeros(3)
+            c[a] = 0.7 * s
+            b = len(pos)
+            e = [np.roll([0.0, 0.2 * s, 0.0], a), np.roll([0.0, 0.0, 0.2 * s], a)]
+            pos += [c - e[0] - e[1], c + e[0] - e[1], c + e[0] + e[1], c - e[0] + e[1]]
+            idx += [[b, b + 1, b + 2], [b, b + 2, b + 3]]
+        s /= 3.0
+    return _rt.HostScene.build(np.array(pos, np.float32), np.array(idx, np.uint32))
+
+
+def centre_rays(n, seed):
+    """Rays that pass close to the nested quads' common centre, so they meet most levels."""
+    rng = np.random.default_rng(seed)
+    rays = np.zeros((n, 8), np.float32)
+    o = rng.random((n, 3)) + 0.5
+    at = rng.random((n, 3)) * 10.0 ** rng.uniform(-20.0, 0.0, (n, 1))
+    rays[:, 0:3], rays[:, 3] = o, 1e30
+    rays[:, 4:7] = (at - o) / np.linalg.norm(at - o, axis=1, keepdims=True)
+    return rays
+
+
+SCENES = {"cornell": _rt.HostScene.cornell, "heightfield": lambda: _rt.HostScene.heightfield(20, 7),
+          "clutter": lambda: _rt.HostScene.clutter(3, 5), "nested": lambda: nested_scene(30),
+          "triangle": lambda: _rt.HostScene.build([[0, 0, 0], [1, 0, 0.2], [0, 1, 0.1]], [[0, 1, 2]])}
+
+
+@pytest.mark.parametrize("watertight", [False, True])
+@pytest.mark.parametrize("scene", sorted(SCENES))
+def test_walk_equals_brute_force(walk, oracle, scene, watertight):
+    hs = SCENES[scene]()
+    sc = oracle.Scene(hs.arrays())
+    rays = ray_set(hs, 4000, 11)
+    want = oracle.bruteforce(sc, rays, watertight=watertight)
+    want_any = oracle.bruteforce(sc, rays, any_hit=True, watertight=watertight)[:, 0]
+    assert 0 < (want[:, 0] >= 0).sum() < len(rays)
+    for leaf in (1, 2, 5, 16):
+        for lds in (10, 1):  # one LDS entry: every deeper one is in the spill stack
+            got, _ = walk(hs, rays, leaf, watertight=watertight, lds=lds)
+            assert np.array_equal(got, want), (leaf, lds, np.nonzero((got != want).any(1))[0][:5])
+            got, _ = walk(hs, rays, leaf, any_hit=True, watertight=watertight, lds=lds)
+            assert np.array_equal(got[:, 0], want_any), (leaf, lds)
+
+
+def test_every_triangle_is_packed_once(walk):
+    for name in sorted(SCENES):
+        hs = SCENES[name]()
+        for leaf in (1, 2, 16):
+            _, n = walk(hs, ray_set(hs, 8, 1), leaf)
+            assert n["tris"] == hs.info()["num_triangles"], (name, leaf)
+
+
+def test_deep_tree_uses_the_spill_stack(walk, oracle):
+    """The walk needs far more entries than any LDS stack holds, and the host's bound covers them."""
+    hs = nested_scene(60)
+    sc, rays = oracle.Scene(hs.arrays()), centre_rays(2000, 3)
+    got, n = walk(hs, rays, 1, lds=10)
+    assert np.array_equal(got, oracle.bruteforce(sc, rays))
+    assert n["used"] > 48
+    got, n = walk(hs, rays, 1, any_hit=True, lds=10)
+    assert np.array_equal(got[:, 0], oracle.bruteforce(sc, rays, any_hit=True)[:, 0])
