@@ -75,15 +75,12 @@ __device__ __forceinline__ void render_tile(const BatchSlot& sl, uint32_t local,
   pt_pixel<WIDE, S>(p, ctx, gx, gy, &c->rays);
 }
 
-// Five waves per SIMD, as the single-scene path tracer (no spill here).
-template <bool WIDE, int S>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_batch_persistent(
-    const BatchSlot* __restrict__ slots, uint32_t numScenes, uint32_t totalTiles, BatchCounters* c, uint2* spillBase,
-    uint32_t spillDepth, uint32_t grab) {
-  __shared__ uint2 stk[WIDE ? S * kTileThreads : 1];
+// The escape walk: one 8x8 tile at a time, each pixel's path where it is needed.
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_batch_persistent_ref(
+    const BatchSlot* __restrict__ slots, uint32_t numScenes, uint32_t totalTiles, BatchCounters* c, uint2*, uint32_t,
+    uint32_t grab) {
   __shared__ uint32_t sBase;
   const int tid = threadIdx.x;
-  uint2* spill = WIDE ? spillBase + ((size_t)blockIdx.x * kTileThreads + tid) * spillDepth : nullptr;
   const uint32_t seed = c->seed;
   for (;;) {
     if (tid == 0) sBase = atomicAdd(&c->tile, grab);
@@ -95,9 +92,59 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5)
     for (uint32_t t = base; t < end; ++t) {
       uint32_t s = 0;
       while (s + 1 < numScenes && slots[s + 1].tileBase <= t) ++s;
-      render_tile<WIDE, S>(slots[s], t - slots[s].tileBase, seed, stk, spill, c);
+      render_tile<false, 16>(slots[s], t - slots[s].tileBase, seed, nullptr, nullptr, c);
     }
   }
+}
+
+// The tiles of one scene for phased_paths, out of the wave's current grab and the
+// ones it takes; stops at the first tile of another scene, which stays the wave's.
+struct SceneTiles {
+  BatchCounters* c;
+  uint32_t totalTiles, grab;
+  uint32_t tile, end;          // the grab: tiles [tile, end)
+  uint32_t sceneBase, sceneEnd;
+  // the wave has a tile (takes the next grab if it must)
+  __device__ bool ready() {
+    if (tile < end) return true;
+    uint32_t v = 0;
+    if ((threadIdx.x & 63) == 0) v = atomicAdd(&c->tile, grab);
+    tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    end = min(totalTiles, tile + grab);
+    return tile < end;
+  }
+  __device__ bool next(uint32_t& chunk) {
+    if (!ready() || tile < sceneBase || tile >= sceneEnd) return false;
+    chunk = tile++ - sceneBase;
+    return true;
+  }
+};
+
+// The wide walk: the paths of one scene after the other's in phases, lanes taking
+// pixels of the scene's next tiles; the wave changes scenes together.  Four waves
+// per SIMD, as the single-scene path tracer.
+template <int S>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_batch_persistent_wide(
+    const BatchSlot* __restrict__ slots, uint32_t numScenes, uint32_t totalTiles, BatchCounters* c, uint2* spillBase,
+    uint32_t spillDepth, uint32_t grab) {
+  __shared__ uint2 stk[S * kTileThreads];
+  uint2* spill = spillBase + ((size_t)blockIdx.x * kTileThreads + threadIdx.x) * spillDepth;
+  SceneTiles source{c, totalTiles, grab, 0u, 0u, 0u, 0u};
+  PtProgram prog{nullptr, c->seed};
+  uint32_t s = 0;
+  while (source.ready()) {
+    while (s + 1 < numScenes && slots[s + 1].tileBase <= source.tile) ++s;  // the wave's tiles only go up
+    const BatchSlot& sl = slots[s];
+    source.sceneBase = sl.tileBase;
+    source.sceneEnd = sl.tileBase + sl.tilesX * sl.tilesY;
+    prog.params = &sl.p;
+    phased_paths<false, S>(sl.p.wide, stk, spill, sl.tilesX * sl.tilesY * kTileThreads, source, (uint32_t)kTileThreads,
+                           prog);
+  }
+  // one atomic per wave
+  uint32_t sum = prog.rays;
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  if (threadIdx.x == 0) atomicAdd(&c->rays, (unsigned long long)sum);
 }
 
 // One scene, one tile per workgroup (the "separate launches" baseline).
@@ -115,8 +162,12 @@ void LaunchTiles(bool persistent, dim3 persistentGrid, const std::vector<BatchSl
                  uint32_t totalTiles, BatchCounters* c, uint2* spill, uint32_t spillDepth, uint32_t grab,
                  hipStream_t stream) {
   if (persistent) {
-    hipLaunchKernelGGL((k_batch_persistent<WIDE, S>), persistentGrid, dim3(kTileThreads), 0, stream, dSlots,
-                       (uint32_t)hSlots.size(), totalTiles, c, spill, spillDepth, grab);
+    if constexpr (WIDE)
+      hipLaunchKernelGGL(k_batch_persistent_wide<S>, persistentGrid, dim3(kTileThreads), 0, stream, dSlots,
+                         (uint32_t)hSlots.size(), totalTiles, c, spill, spillDepth, grab);
+    else
+      hipLaunchKernelGGL(k_batch_persistent_ref, persistentGrid, dim3(kTileThreads), 0, stream, dSlots,
+                         (uint32_t)hSlots.size(), totalTiles, c, spill, spillDepth, grab);
     return;
   }
   for (size_t i = 0; i < hSlots.size(); ++i) {
@@ -162,7 +213,7 @@ struct gpugi_batch {
   uint32_t totalTiles = 0;
   int kernel = GPUGI_KERNEL_WIDE;
   int grab = 2;
-  int gridMul = 2;
+  int gridMul = 4;  // 5.9 ms a frame of the 16 benchmark scenes; 6.7 at 3, 8.4 at 2
   int stackDepth = 16;     // one of kBatchStacks
   int residentRef = 1;     // resident blocks per CU of the reference-walk kernel
   int residentWide[3] = {1, 1, 1};  // ... of the wide kernel per kBatchStacks entry
@@ -395,15 +446,15 @@ int gpugi_batch_finalize(gpugi_batch* b) {
   for (size_t i = 0; i < b->hSlots.size(); ++i) b->hSlots[i].p.accum = b->dAccum + b->accumOffset[i];
   BHIP(b, hipMalloc((void**)&b->dSlots, b->hSlots.size() * sizeof(BatchSlot)));
   BHIP(b, hipMemcpy(b->dSlots, b->hSlots.data(), b->hSlots.size() * sizeof(BatchSlot), hipMemcpyHostToDevice));
-  const void* wideKernels[3] = {(const void*)&k_batch_persistent<true, 16>, (const void*)&k_batch_persistent<true, 24>,
-                                (const void*)&k_batch_persistent<true, 32>};
+  const void* wideKernels[3] = {(const void*)&k_batch_persistent_wide<16>, (const void*)&k_batch_persistent_wide<24>,
+                                (const void*)&k_batch_persistent_wide<32>};
   for (int i = 0; i < 3; ++i) {
     int r = 0;
     BHIP(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, wideKernels[i], kTileThreads, 0));
     b->residentWide[i] = std::max(1, r);
   }
   int r = 0;
-  BHIP(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)&k_batch_persistent<false, 16>, kTileThreads, 0));
+  BHIP(b, hipOccupancyMaxActiveBlocksPerMultiprocessor(&r, (const void*)&k_batch_persistent_ref, kTileThreads, 0));
   b->residentRef = std::max(1, r);
   b->finalized = true;
   return gpugi_batch_reset(b, 0);

@@ -51,7 +51,7 @@ struct gpugi_ctx {
   void* dCounters = nullptr;  // [0] ray counter, [1] error flag, [2] hit count
   void* dWideQueue = nullptr;  // the wide trace kernel's batch counters
   size_t spillBytes = 0;
-  uint32_t wideMaxStack = 0, wideMaxPending = 0;
+  uint32_t wideMaxStack = 0, wideMaxPending = 0, wideNumNodes = 0;
   int wideLeaf = 2;     // triangles per merged wide leaf
   int wideStack = 10;   // LDS stack entries per lane of the trace kernel
   int wideRefill = 8;   // idle lanes that trigger a wave-level ray refill
@@ -263,6 +263,7 @@ int RebuildWide(gpugi_ctx* ctx) {
                            hipMemcpyHostToDevice));
   ctx->wideMaxStack = wide.maxStack;
   ctx->wideMaxPending = wide.maxPending;
+  ctx->wideNumNodes = (uint32_t)wide.nodes.size();
   ctx->hasWide = true;
   return GPUGI_OK;
 }
@@ -761,6 +762,7 @@ static DrawParams MakeDrawParams(gpugi_ctx* ctx, uint32_t frame_seed) {
   p.ref = MakeRef(ctx);
   p.wide = MakeWide(ctx, kWideLdsStack);
   p.useWide = ctx->hasWide && ctx->integratorKernel != GPUGI_KERNEL_REFERENCE;
+  p.wideNodes = ctx->wideNumNodes;
   p.materials = (const gpugi_material*)ctx->dMats;
   p.lights = (const gpugi_light_sample*)ctx->dLights;
   p.numLights = ctx->numLights;

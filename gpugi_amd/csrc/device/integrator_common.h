@@ -10,6 +10,7 @@ namespace gpugi {
 
 constexpr int kTile = 8;                 // local size 8x8 of pathtracer.comp:14-15
 constexpr int kTileThreads = kTile * kTile;
+constexpr int kLull = 4;  // phased_paths: trace passes go on while this many lanes a pass finish their rays
 
 // Closest / any hit through either traversal.  The wide walk needs a per-lane
 // LDS stack (S x 64 entries per block) and a global spill slice.
@@ -45,7 +46,7 @@ __device__ __forceinline__ void persistent_items(uint32_t numItems, uint32_t* qu
       if (avail < nidle) {
         uint32_t v = 0;
         if (lane == 0) v = atomicAdd(queue, 1u);
-        v = (uint32_t)__shfl((int)v, 0);
+        v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
         if (v < chunks) next = v;
       }
       if (!live) {
@@ -83,6 +84,131 @@ __device__ __forceinline__ void tile_pixel(uint32_t item, int width, int& gx, in
   const uint32_t tilesX = (uint32_t)width / kTile, tile = item / kTileThreads, k = item % kTileThreads;
   gx = (int)((tile % tilesX) * kTile + k % kTile);
   gy = (int)((tile / tilesX) * kTile + k / kTile);
+}
+
+// What a path does next (a program of phased_paths).
+enum PathNext {
+  kPathEnds,     // the path is finished
+  kPathCloses,   // the closest hit of its ray (o, d)
+  kPathOccludes  // whether its light ray (lo, ld, ltmax) is blocked
+};
+
+// Chunks of consecutive items for phased_paths: [0, chunks) from *queue (zeroed
+// before the launch).  next() is called by the whole wave.
+struct QueueChunks {
+  uint32_t* queue;
+  uint32_t chunks;
+  __device__ bool next(uint32_t& chunk) {
+    uint32_t v = 0;
+    if ((threadIdx.x & 63) == 0) v = atomicAdd(queue, 1u);
+    chunk = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    return chunk < chunks;
+  }
+};
+
+// Work items [0, numItems) for a persistent one-wave block over the wide BVH, in
+// phases: every lane carries a path of its own, and the lanes of the wave are in
+// different rays of different bounces, but each turn of the loop runs one kind
+// of pass over the lanes that wait for it:
+//   trace    a box or leaf pass (trace_wide.h) of all lanes with a ray, closest
+//            and light rays alike;
+//   shade    prog.shade(slot, t, b_y, b_z) for the lanes whose closest hit is known;
+//   resolve  prog.resolve(blocked) for the lanes whose light ray is done, and new
+//            items (prog.begin(item)) for the lanes without one.
+// shade and resolve say what the path does next; prog.finish() ends an item.
+// Shading is long, so it waits until as many lanes wait for it as trace and fewer
+// than kLull rays end with a trace pass; resolving waits for an eighth of the
+// lanes at work.  A wave therefore neither traces until its longest ray ends
+// before it shades nor shades for a few lanes at a time.  What an item computes
+// does not depend on when its passes run.  Items come in chunks of `lanes` from
+// `source`; the first `lanes` lanes of the wave carry them.
+//
+// Bound by VALU issue (1.0 wave-instructions per CU and cycle).  Against tracing
+// each ray where it is needed (persistent_items), whose passes run with the
+// lanes of every other phase masked off: 35 lanes active instead of 16, path
+// tracing the 5,120,016-triangle room at 1920x1080 (path length 8) 9.5 -> 6.5 ms
+// a frame.  Four waves per SIMD (128 VGPRs): five spill 112 bytes a lane and
+// take 6.6 ms.
+template <bool WT, int S, class Source, class Prog>
+__device__ __forceinline__ void phased_paths(const WideScene& ws, uint2* lds, uint2* spill, uint32_t numItems,
+                                             Source& source, uint32_t lanes, Prog& prog) {
+  enum { kIdle, kTraces, kShades, kResolves, kUnused };
+  const WideStack stk{as_lds(lds), (int)threadIdx.x, spill, 1u};
+  const uint64_t below = (1ull << (threadIdx.x & 63)) - 1ull;
+  // wave-uniform: the chunk being handed out and how many of its items are gone
+  uint32_t cur = 0, pos = lanes;
+  bool exhausted = false;
+  uint32_t mode = (threadIdx.x & 63) < lanes ? kIdle : kUnused;
+  WideState st;
+  for (;;) {
+    // Trace passes until enough lanes wait for another pass.  (A loop of its own:
+    // its turns carry the traversal's registers only.)
+    bool shade, other;
+    for (int lastTraces = 0;;) {
+      const uint64_t traces = __ballot(mode == kTraces);
+      const int numTraces = __popcll(traces), numShades = __popcll(__ballot(mode == kShades));
+      const int numIdle = __popcll(__ballot(mode == kIdle));
+      const int live = exhausted ? (int)lanes - numIdle : (int)lanes;
+      const int numOther = live - numTraces - numShades;
+      other = numOther > 0 && (8 * numOther >= live || numTraces == 0);
+      shade = numShades > 0 && ((numShades >= numTraces && lastTraces - numTraces < kLull) || numTraces == 0);
+      if (other || shade || live == 0) break;
+      lastTraces = numTraces;
+      const bool leafPass = wide_choose_leaf_pass(traces, st, (numTraces + 7) / 8);
+      if (mode == kTraces && wide_pass<kWideMixed, kTileThreads, S, WT>(ws, st, leafPass, stk))
+        mode = st.anyHit ? kResolves : kShades;
+    }
+    if (!other && !shade) break;  // no lane has an item
+    PathNext next = kPathEnds;
+    bool advanced = false;  // the lane's path has just got to its next ray or its end
+    if (shade) {
+      if (mode == kShades) {
+        next = prog.shade(st.bestSlot, st.tbest, st.bu, st.bv);
+        advanced = true;
+      }
+    }
+    if (other) {
+      if (mode == kResolves) {
+        next = prog.resolve(st.bestSlot >= 0);
+        advanced = true;
+      }
+      if (!exhausted) {
+        const uint64_t idle = __ballot(mode == kIdle);
+        const uint32_t nidle = (uint32_t)__popcll(idle), avail = lanes - pos;
+        uint32_t chunk = 0;
+        const bool more = avail < nidle && source.next(chunk);
+        if (mode == kIdle) {
+          const uint32_t rank = (uint32_t)__popcll(idle & below);
+          uint32_t item = numItems;
+          if (rank < avail) item = cur * lanes + pos + rank;
+          else if (more) item = chunk * lanes + (rank - avail);
+          if (item < numItems) {
+            next = prog.begin(item);
+            advanced = true;
+          }
+        }
+        if (avail >= nidle) {
+          pos += nidle;
+        } else if (more) {
+          cur = chunk;
+          pos = nidle - avail;
+        } else {
+          exhausted = true;
+        }
+      }
+    }
+    if (advanced) {
+      if (next == kPathEnds) {
+        prog.finish();
+        mode = kIdle;
+      } else {
+        const bool any = next == kPathOccludes;
+        wide_init<WT>(st, any ? prog.lo : prog.o, any ? prog.ld : prog.d, any ? prog.ltmax : gg::kRayMax);
+        st.anyHit = any;
+        mode = kTraces;
+      }
+    }
+  }
 }
 
 struct ClosestHit {
@@ -251,18 +377,24 @@ __device__ __forceinline__ void pt_begin(const DrawParams& p, PtPath& s, int gx,
   s.d = gg::primary_direction(j0, j1, gx, gy, p.width, p.height, U, V, W);
 }
 
-// One bounce of the path (the loop body of pathtracer.comp).  Returns true
-// when the path has ended; s.color is then final.
-template <bool WIDE, int S = kWideLdsStack>
-__device__ __forceinline__ bool pt_bounce(const DrawParams& p, const TraceCtx& c, PtPath& s) {
-  if (s.bounce >= p.maxPathLength) return true;
-  const float lightSampleWeight = (float)p.numLights / 1.0f;
-  const ClosestHit h = trace_closest<WIDE, S>(c, s.o, s.d);
+// The light sample of a bounce: s.color gains `unblocked` if its ray is not
+// blocked, else `blocked` (a zero, or NaN where the throughput is not finite).
+struct PtLight {
+  NeeSample ns;
+  gg::V3 unblocked, blocked;
+};
+
+// One bounce of the path (the loop body of pathtracer.comp) at the closest hit h
+// of its ray, up to the ray of its light sample (l.ns.test: there is one to
+// trace).  Returns whether the path goes on with (s.o, s.d) once l's term is added.
+__device__ __forceinline__ bool pt_shade(const DrawParams& p, PtPath& s, const ClosestHit& h, PtLight& l) {
+  l.ns.test = false;
   if (!h.hit) {
     // environment on a miss (pathtracer.comp:56-58); black by default (renderersystem.cpp:39-47)
     s.color = s.color + s.throughput * (p.env ? env_radiance(p.env, p.envSize, s.d) : gg::v3s(0.0f));
-    return true;
+    return false;
   }
+  const float lightSampleWeight = (float)p.numLights / 1.0f;
   s.o = s.o + h.t * s.d;
   const gg::V3 n = shading_normal(p.ref.vinfo, h.tri, h.bary);
   const MaterialData m = load_material_hit(p.materials, p.tex, p.ref.vinfo, h.tri, h.bary);
@@ -273,8 +405,10 @@ __device__ __forceinline__ bool pt_bounce(const DrawParams& p, const TraceCtx& c
   s.didNEE = m.refl[3] < 500.0f;
   if (spl < 0 || s.bounce + 1 == spl) {
     const int sampleIndex = (int)(gg::xorshift32(s.seed) % p.numLights);
-    const gg::V3 radiance = estimate_direct_light<WIDE, S>(c, s.o, n, sampleIndex, s.d, m, s.didNEE);
-    s.color = s.color + radiance * s.throughput * lightSampleWeight;
+    l.ns = nee_sample(p, s.o, n, sampleIndex, s.d, m, s.didNEE);
+    l.blocked = gg::v3s(0.0f) * s.throughput * lightSampleWeight;
+    l.unblocked = l.ns.value * s.throughput * lightSampleWeight;
+    if (!l.ns.test) s.color = s.color + l.blocked;
   }
   gg::V3 tp = gg::v3s(1.0f);
   float pdf;
@@ -284,11 +418,23 @@ __device__ __forceinline__ bool pt_bounce(const DrawParams& p, const TraceCtx& c
   s.throughput = s.throughput * tp;
   if (s.bounce >= p.rrStartDepth) {  // Russian roulette (pathtracer.comp:99-104) from rrStartDepth on
     const float q = gg::saturate(gg::luminance(tp));
-    if (gg::random01(s.seed) >= q) return true;
+    if (gg::random01(s.seed) >= q) return false;
     s.throughput = s.throughput / q;
   }
   ++s.bounce;
-  return s.bounce >= p.maxPathLength;
+  return s.bounce < p.maxPathLength;
+}
+
+// The whole bounce with its rays traced here.  Returns true when the path has
+// ended; s.color is then final.
+template <bool WIDE, int S = kWideLdsStack>
+__device__ __forceinline__ bool pt_bounce(const DrawParams& p, const TraceCtx& c, PtPath& s) {
+  if (s.bounce >= p.maxPathLength) return true;
+  const ClosestHit h = trace_closest<WIDE, S>(c, s.o, s.d);
+  PtLight l;
+  const bool goesOn = pt_shade(p, s, h, l);
+  if (l.ns.test) s.color = s.color + (trace_any<WIDE, S>(c, l.ns.o, l.ns.dir, l.ns.len) ? l.blocked : l.unblocked);
+  return !goesOn;
 }
 
 // Adds vec4(color, 0) to the pixel's accumulation entry.
@@ -297,6 +443,77 @@ __device__ __forceinline__ void pt_finish(const DrawParams& p, const PtPath& s, 
   const float4 v = *px;
   *px = make_float4(s.color.x + v.x, s.color.y + v.y, s.color.z + v.z, 0.0f + v.w);
 }
+
+// The path tracer's items for phased_paths: the pixels of all 8x8 tiles.
+struct PtProgram {
+  const DrawParams* params;
+  uint32_t frameSeed;
+  gg::V3 o, d, lo, ld;
+  float ltmax;
+  gg::V3 color, throughput, unblocked;
+  uint32_t seed, pixel;
+  int bounce;
+  bool didNEE, goesOn, blockedNaN[3];
+  uint32_t rays = 0;  // traced by this lane
+
+  __device__ PathNext begin(uint32_t item) {
+    const DrawParams& p = *params;
+    int gx, gy;
+    tile_pixel(item, p.width, gx, gy);
+    PtPath s;
+    pt_begin(p, s, gx, gy, frameSeed);
+    o = s.o;
+    d = s.d;
+    color = s.color;
+    throughput = s.throughput;
+    seed = s.seed;
+    bounce = s.bounce;
+    didNEE = s.didNEE;
+    pixel = (uint32_t)gy * (uint32_t)p.width + (uint32_t)gx;
+    if (p.maxPathLength <= 0) return kPathEnds;
+    ++rays;
+    return kPathCloses;
+  }
+  __device__ PathNext shade(int slot, float t, float by, float bz) {
+    PtPath s{color, throughput, o, d, seed, bounce, didNEE};
+    PtLight l;
+    goesOn = pt_shade(*params, s, closest_from_record(*params, slot, t, by, bz), l);
+    color = s.color;
+    throughput = s.throughput;
+    o = s.o;
+    d = s.d;
+    seed = s.seed;
+    bounce = s.bounce;
+    didNEE = s.didNEE;
+    if (l.ns.test) {
+      lo = l.ns.o;
+      ld = l.ns.dir;
+      ltmax = l.ns.len;
+      unblocked = l.unblocked;
+      blockedNaN[0] = l.blocked.x != l.blocked.x;
+      blockedNaN[1] = l.blocked.y != l.blocked.y;
+      blockedNaN[2] = l.blocked.z != l.blocked.z;
+      ++rays;
+      return kPathOccludes;
+    }
+    return more();
+  }
+  __device__ PathNext resolve(bool blocked) {
+    color.x += blocked ? (blockedNaN[0] ? NAN : 0.0f) : unblocked.x;
+    color.y += blocked ? (blockedNaN[1] ? NAN : 0.0f) : unblocked.y;
+    color.z += blocked ? (blockedNaN[2] ? NAN : 0.0f) : unblocked.z;
+    return more();
+  }
+  __device__ PathNext more() {
+    rays += goesOn ? 1u : 0u;
+    return goesOn ? kPathCloses : kPathEnds;
+  }
+  __device__ void finish() {
+    float4* px = &params->accum[pixel];
+    const float4 v = *px;
+    *px = make_float4(color.x + v.x, color.y + v.y, color.z + v.z, 0.0f + v.w);
+  }
+};
 
 // The whole path of pixel (gx, gy) on the calling lane.  rays (optional)
 // counts the rays this path traced.

@@ -16,6 +16,7 @@ struct DrawParams {
   RefScene ref;
   WideScene wide;
   bool useWide = false;
+  uint32_t wideNodes = 0;                 // nodes of the wide BVH
   const gpugi_material* materials = nullptr;
   const gpugi_light_sample* lights = nullptr;
   uint32_t numLights = 0;
@@ -71,14 +72,32 @@ struct IntegratorState {
   uint32_t* lastTotal = nullptr;    // device NumLightCacheEntries of the last BPT draw
   uint32_t* queue = nullptr;        // work counter of the persistent integrator kernels
   std::map<const void*, uint32_t> residentBlocks;  // per kernel: resident one-wave blocks on the device
+  uint32_t simds = 0;               // SIMDs on the device (EnsureSimds)
 };
 
 // Zeroes st->queue on `stream` and sizes the grid of one-wave blocks for a
 // persistent_items kernel: the blocks resident on the device, at most one per
 // 64 items (resident), or one per 64 items, so that blocks rather than lanes
 // take new work (the light paths, whose splats into the image prefer it).
+// lanes (phased_paths kernels): the lanes of a block that carry items, fewer
+// than 64 (but 16 at least) while that leaves no SIMD two blocks: an image that
+// small is bound by the latency of its longest wave, and fewer paths a wave
+// shorten it.  Measured (room of 400 spheres, 64 x 64 and 128 x 128 pixels, per
+// frame): 340 and 400 us against 416 and 449 with 64 lanes; 16 lanes at 256 x 256,
+// four blocks a SIMD, take 528 against 465.
+constexpr uint32_t kPhasedMinLanes = 16;
 hipError_t PersistentGrid(IntegratorState* st, const void* kernel, size_t items, uint32_t* blocks,
-                          hipStream_t stream, bool resident = true);
+                          hipStream_t stream, bool resident = true, uint32_t* lanes = nullptr);
+// Whether the paths of `items` pixels stay in step: at most one wave per SIMD
+// (no lane gets a second pixel) in a tree of at most kInStepNodes nodes, whose
+// rays all end after a few passes.  Such images are faster with each ray traced
+// where it is needed than in phases: 220 against 251 us a frame in the Cornell
+// room, 203 against 223 on a 64 x 64 heightfield (1,000 nodes), both 256 x 256
+// pixels; with 2,600 nodes (room of 16 spheres) phases win, 260 against 280, and
+// so they do in the Cornell room at 1024 x 1024, 704 against 729.
+constexpr uint32_t kInStepNodes = 1536;
+hipError_t EnsureSimds(IntegratorState* st);
+bool PathsInStep(const IntegratorState* st, const DrawParams& p, size_t items);
 
 // Grows a device buffer to at least `bytes` (contents are not preserved).
 inline hipError_t EnsureBuffer(void** buf, size_t* cap, size_t bytes) {

@@ -51,6 +51,9 @@ constexpr uint32_t kWideNoNode = 0xffffffffu;
 constexpr uint32_t kWideLeafEntry = 0x80000000u;
 constexpr uint32_t kWideBoundMask = 0xfff80000u;
 
+// What the lanes of a wave trace: closest hits, any hits, or either, by WideState::anyHit.
+enum WideQuery { kWideClosest = 0, kWideAny = 1, kWideMixed = 2 };
+
 struct WideResult {
   float t;     // final ray length (tmax on a miss)
   int slot;    // reference slot index, -1 on a miss, -2 on stack overflow
@@ -91,8 +94,9 @@ struct WideState {
   uint32_t leafNode[2];  // the pending leaf groups' nodes
   uint32_t leafMask;     // their hit leaves' slots, 8 bits each; 0: none, below 256: the first only
   int sp;
-  bool found;
-  WtRay wr;  // watertight mode only
+  bool found;   // kWideAny only
+  bool anyHit;  // kWideMixed only; such a ray has found an occluder once bestSlot >= 0
+  WtRay wr;     // watertight mode only
 };
 
 // 1/d by v_rcp_f32 (within 1 ulp): a reciprocal with relative error
@@ -148,10 +152,12 @@ __device__ __forceinline__ uint32_t wide_child(uint32_t first, uint32_t inner, u
 
 // Which of the waiting slots (not 0) is visited next: the nearest one if it waits
 // (if it is not a leaf or gone already), else the first; any hit: the last.
-template <bool ANY>
-__device__ __forceinline__ uint32_t wide_next(uint32_t waiting, uint32_t nearest) {
-  if (ANY) return 31u - (uint32_t)__builtin_clz(waiting);
-  return (waiting >> nearest) & 1u ? nearest : (uint32_t)__builtin_ctz(waiting);
+template <int Q>
+__device__ __forceinline__ uint32_t wide_next(const WideState& st, uint32_t waiting, uint32_t nearest) {
+  const uint32_t last = 31u - (uint32_t)__builtin_clz(waiting);
+  if (Q == kWideAny) return last;
+  const uint32_t closest = (waiting >> nearest) & 1u ? nearest : (uint32_t)__builtin_ctz(waiting);
+  return Q == kWideMixed && st.anyHit ? last : closest;
 }
 
 // Puts an entry on the stack; false if it would overflow (impossible when the
@@ -177,7 +183,7 @@ __device__ __forceinline__ bool wide_hold(WideState& st, uint32_t node, uint32_t
 
 // Box pass for a lane with st.node != kWideNoNode.  Returns false if the stack
 // would overflow.
-template <bool ANY, int B, int S>
+template <int Q, int B, int S>
 __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, const WideStack& stk) {
   const gg::V3 o = st.o;
   const uint32_t nodeIndex = st.node;
@@ -236,7 +242,7 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
                                       plane_fma(nz, h, Az24, bnz)), 0.0f);
       const float tfar = fminf(fminf(fminf(plane_fma(fx, h, Ax24, bfx), plane_fma(fy, h, Ay24, bfy)),
                                      plane_fma(fz, h, Az24, bfz)), tbScaled);
-      if (ANY) {
+      if (Q == kWideAny) {
         misses = __builtin_amdgcn_alignbit(misses, __float_as_uint(tfar - tnear), 31);
       } else {
         keys[k] = tnear <= tfar ? (__float_as_uint(tnear) & ~7u) | (uint32_t)k : 0xffffffffu;
@@ -245,7 +251,7 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
     }
   }
   uint32_t first = 0xffffffffu;  // the smallest key
-  if (!ANY) {
+  if (Q != kWideAny) {
 #pragma unroll
     for (int k = 0; k < kWideArity; ++k) first = min(first, keys[k]);
   }
@@ -255,12 +261,12 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
   bool fits = true;
   st.node = kWideNoNode;
   if (waiting != 0u) {
-    const uint32_t next = wide_next<ANY>(waiting, first & 7u);
+    const uint32_t next = wide_next<Q>(st, waiting, first & 7u);
     st.node = wide_child(q1.x, inner, next);
     waiting &= ~(1u << next);
     if (waiting != 0u) {
       uint32_t e = waiting | (inner << 8);
-      if (!ANY) {
+      if (Q != kWideAny) {
         // the second smallest key: a distance, since two children or more are hit, and
         // no larger than those of the children that wait
         uint32_t a = keys[0], second = 0xffffffffu;
@@ -275,7 +281,7 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
     }
   }
   if (leaves != 0u && !wide_hold(st, nodeIndex, leaves))
-    fits = wide_push<B, S>(s, st, stk, make_uint2(nodeIndex | kWideLeafEntry, leaves | (ANY ? 0u : first & kWideBoundMask))) &&
+    fits = wide_push<B, S>(s, st, stk, make_uint2(nodeIndex | kWideLeafEntry, leaves | (Q == kWideAny ? 0u : first & kWideBoundMask))) &&
            fits;
   if (!fits) {
     atomicOr(s.errorFlag, 1u);
@@ -288,7 +294,7 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
 // the first group.  One leaf a pass: a lane with several does not hold the
 // others' next passes (2^24 diffuse rays on the heightfield: 2460 us with all of
 // a lane's leaves in one pass, 2246 us with one).
-template <bool ANY, bool WT>
+template <int Q, bool WT>
 __device__ __forceinline__ void wide_leaf(const WideScene& s, WideState& st) {
   const gg::V3 o = st.o, d = st.d;
   // {firstChild, firstTri, ends} of the group's node
@@ -328,7 +334,7 @@ __device__ __forceinline__ void wide_leaf(const WideScene& s, WideState& st) {
       t = gg::dot(nn, e2);
       ok = t > 0.0001f && bx >= 0.0f && by >= 0.0f && bz >= 0.0f;
     }
-    if (ANY) {
+    if (Q == kWideAny) {
       if (ok && t < st.tbest) {
         st.found = true;
         return;
@@ -345,7 +351,7 @@ __device__ __forceinline__ void wide_leaf(const WideScene& s, WideState& st) {
 // For a lane without a next node: pops entries still in front of the closest
 // hit until one yields a node, or a leaf group finds both pending slots taken
 // (the entry stays), or the stack is empty.
-template <bool ANY, int B, int S>
+template <int Q, int B, int S>
 __device__ __forceinline__ void wide_pop(WideState& st, const WideStack& stk) {
   const float tb = st.tbest * 1.00000095f;  // entry distances are lower bounds with this slack
   int sp = st.sp;
@@ -355,7 +361,7 @@ __device__ __forceinline__ void wide_pop(WideState& st, const WideStack& stk) {
     uint2 e;
     if (top < S) e = stk.lds[top * B + stk.tid];
     else e = stk.spill[(size_t)(top - S) * stk.spillStride];
-    if (!ANY && __uint_as_float(e.y & kWideBoundMask) > tb) {
+    if (Q != kWideAny && __uint_as_float(e.y & kWideBoundMask) > tb) {
       sp = top;
       continue;
     }
@@ -364,7 +370,7 @@ __device__ __forceinline__ void wide_pop(WideState& st, const WideStack& stk) {
       sp = top;
       continue;
     }
-    const uint32_t next = wide_next<ANY>(e.y & 0xffu, (e.y >> 16) & 7u);  // a node entry has a waiting child
+    const uint32_t next = wide_next<Q>(st, e.y & 0xffu, (e.y >> 16) & 7u);  // a node entry has a waiting child
     node = wide_child(e.x, (e.y >> 8) & 0xffu, next);
     e.y &= ~(1u << next);
     if ((e.y & 0xffu) == 0u) sp = top;
@@ -385,18 +391,19 @@ __device__ __forceinline__ bool wide_choose_leaf_pass(uint64_t working, const Wi
 }
 
 // One pass for a working lane.  Returns true when the ray is finished.
-template <bool ANY, int B, int S, bool WT>
+template <int Q, int B, int S, bool WT>
 __device__ __forceinline__ bool wide_pass(const WideScene& s, WideState& st, bool leafPass, const WideStack& stk) {
   if (leafPass) {
     if (st.leafMask == 0u) return false;  // still traversing; unaffected by this pass
-    wide_leaf<ANY, WT>(s, st);
-    if (ANY && st.found) return true;
+    wide_leaf<Q, WT>(s, st);
+    if (Q == kWideAny && st.found) return true;
+    if (Q == kWideMixed && st.anyHit && st.bestSlot >= 0) return true;
   } else {
     if (st.node == kWideNoNode) return false;  // waiting for a leaf pass
-    if (!wide_visit<ANY, B, S>(s, st, stk)) return true;  // overflow, slot -2
+    if (!wide_visit<Q, B, S>(s, st, stk)) return true;  // overflow, slot -2
   }
   if (st.node == kWideNoNode) {
-    wide_pop<ANY, B, S>(st, stk);
+    wide_pop<Q, B, S>(st, stk);
     return st.node == kWideNoNode && st.leafMask == 0u;
   }
   return false;

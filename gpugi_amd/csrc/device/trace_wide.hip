@@ -75,7 +75,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_t
       if (avail < nidle) {  // take the XCD's next batch
         uint32_t v = 0;
         if (lane == 0) v = atomicAdd(counter, 1u);
-        v = (uint32_t)__shfl((int)v, 0);
+        v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
         if (v < bEnd - bBegin) next = bBegin + v;
       }
       if (!active) {

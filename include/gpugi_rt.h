@@ -644,7 +644,7 @@ int gpugi_batch_finalize(gpugi_batch* batch);
  * the 8-wide BVH), tiles taken per queue access, the persistent grid in
  * quarters of full residency (1..16) and the wide walk's LDS stack entries
  * per lane (16, 24 or 32; deeper entries spill to global memory; the escape
- * walk ignores it).  Defaults: WIDE, 2, 2, 16. */
+ * walk ignores it).  Defaults: WIDE, 2, 4, 16. */
 int gpugi_batch_config(gpugi_batch* batch, int kernel, int tiles_per_grab, int grid_multiplier, int stack_depth);
 /* Clears every accumulation buffer and the ray counter; the next frame is frame_index. */
 int gpugi_batch_reset(gpugi_batch* batch, uint32_t frame_index);
