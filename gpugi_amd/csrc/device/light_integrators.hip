@@ -33,22 +33,27 @@ __device__ __forceinline__ void splat_add(float* p, float v) {
 
 // ProjectToScreen without DEPTH_BUFFER_OCCLUSION_TEST / CHAINED_MIS and with
 // the box reconstruction filter (screenreproject.glsl:55-227).
-template <bool WIDE>
-__device__ __forceinline__ void project_to_screen(const TraceCtx& c, gg::V3 rayO, gg::V3 rayD, gg::V3 gN,
-                                                  gg::V3 sN, const MaterialData& m, gg::V3 tp, bool computeMIS) {
-  const DrawParams& p = *c.p;
+// Returns whether there is a camera ray to trace; if it is not blocked the
+// splat is added (add_splat).
+struct CameraSplat {
+  gg::V3 o, d, color;
+  float tmax;
+  uint32_t pixel;
+};
+__device__ __forceinline__ bool project_to_screen(const DrawParams& p, gg::V3 rayO, gg::V3 rayD, gg::V3 gN, gg::V3 sN,
+                                                  const MaterialData& m, gg::V3 tp, bool computeMIS, CameraSplat& out) {
   const gg::V3 U = gg::v3(p.camera.u[0], p.camera.u[1], p.camera.u[2]);
   const gg::V3 V = gg::v3(p.camera.v[0], p.camera.v[1], p.camera.v[2]);
   const gg::V3 W = gg::v3(p.camera.w[0], p.camera.w[1], p.camera.w[2]);
   const gg::V3 cp = gg::v3(p.camera.position[0], p.camera.position[1], p.camera.position[2]);
   gg::V3 crd = cp - rayO;
   const float camViewDotRay = -gg::dot(W, crd);
-  if (!(camViewDotRay > 0.0f)) return;
+  if (!(camViewDotRay > 0.0f)) return false;
   float sx = -gg::dot(U, crd) / camViewDotRay;
   float sy = -gg::dot(V, crd) / camViewDotRay;
   sx = sx / gg::dot(U, U);
   sy = sy / gg::dot(V, V);
-  if (!(sx >= -1.0f && sx < 1.0f && sy > -1.0f && sy <= 1.0f)) return;
+  if (!(sx >= -1.0f && sx < 1.0f && sy > -1.0f && sy <= 1.0f)) return false;
   const float cameraDistSq = gg::dot(crd, crd);
   const float cameraDist = sqrtf(cameraDistSq);
   crd = crd / cameraDist;
@@ -71,10 +76,18 @@ __device__ __forceinline__ void project_to_screen(const TraceCtx& c, gg::V3 rayO
   // Splats outside the image are dropped, as image atomics outside the image
   // are, and a splat of exactly zero changes nothing (the accumulated sums
   // are never -0): neither needs the camera ray, which is traced last.
-  if (ix < 0 || ix >= p.width || iy < 0 || iy >= p.height) return;
-  if (color.x == 0.0f && color.y == 0.0f && color.z == 0.0f) return;
-  if (trace_any<WIDE>(c, co, crd, cameraDist)) return;
-  float* px = reinterpret_cast<float*>(&p.accum[(size_t)iy * p.width + ix]);
+  if (ix < 0 || ix >= p.width || iy < 0 || iy >= p.height) return false;
+  if (color.x == 0.0f && color.y == 0.0f && color.z == 0.0f) return false;
+  out.o = co;
+  out.d = crd;
+  out.tmax = cameraDist;
+  out.color = color;
+  out.pixel = (uint32_t)iy * (uint32_t)p.width + (uint32_t)ix;
+  return true;
+}
+
+__device__ __forceinline__ void add_splat(const DrawParams& p, uint32_t pixel, gg::V3 color) {
+  float* px = reinterpret_cast<float*>(&p.accum[pixel]);
   splat_add(px + 0, color.x);
   splat_add(px + 1, color.y);
   splat_add(px + 2, color.z);
@@ -146,14 +159,15 @@ __device__ __forceinline__ void lt_begin(const DrawParams& p, LtPath& s, uint32_
   s.bounce = 0;
 }
 
-// One bounce; true when the path has ended.
-template <bool WIDE, int MODE>
-__device__ __forceinline__ bool lt_bounce(const DrawParams& p, const TraceCtx& c, LtPath& s,
-                                          LightCacheEntryDev* __restrict__ staging) {
+// One bounce at the closest hit h of the path's ray, up to the ray of its camera
+// connection (splats: there is one to trace, for `splat`).  Returns whether the
+// path goes on with (s.o, s.d).
+template <int MODE>
+__device__ __forceinline__ bool lt_shade(const DrawParams& p, LtPath& s, const ClosestHit& h,
+                                         LightCacheEntryDev* __restrict__ staging, bool& splats, CameraSplat& splat) {
+  splats = false;
+  if (!h.hit) return false;
   const int i = s.bounce;
-  if (i >= p.maxPathLength) return true;
-  const ClosestHit h = trace_closest<WIDE>(c, s.o, s.d);
-  if (!h.hit) return true;
   s.o = s.o + h.t * s.d;
   const gg::V3 sN = shading_normal(p.ref.vinfo, h.tri, h.bary);
   const float2 uv = hit_texcoord(p.ref.vinfo, h.tri, h.bary);
@@ -169,7 +183,7 @@ __device__ __forceinline__ bool lt_bounce(const DrawParams& p, const TraceCtx& c
   }
   // the camera connection closes a path of i + 1 bounces (lighttracer.comp:133-157)
   if (MODE != kModeBptWarmup && (p.specificPathLength < 0 || i + 1 == p.specificPathLength))
-    project_to_screen<WIDE>(c, s.o, s.d, h.geoNormal, sN, m, s.tp, MODE == kModeBptLight);
+    splats = project_to_screen(p, s.o, s.d, h.geoNormal, sN, m, s.tp, MODE == kModeBptLight, splat);
   gg::V3 t1 = gg::v3s(1.0f);
   float pdf;
   bool diffuse;
@@ -178,23 +192,90 @@ __device__ __forceinline__ bool lt_bounce(const DrawParams& p, const TraceCtx& c
   s.tp = s.tp * t1;
   if (i >= p.rrStartDepth) {  // Russian roulette (lighttracer.comp:183-188) from rrStartDepth on
     const float q = gg::saturate(gg::luminance(t1));
-    if (gg::random01(s.seed) >= q) return true;
+    if (gg::random01(s.seed) >= q) return false;
     s.tp = s.tp / q;
   }
   s.d = nd;
   s.o = s.o + s.d * gg::kRayHitEpsilon;
   ++s.bounce;
-  return s.bounce >= p.maxPathLength;
+  return s.bounce < p.maxPathLength;
 }
 
-// All numPaths light paths with path regeneration (persistent_items).  Five
-// waves per SIMD (at most 96 VGPRs): the BPT light pass would otherwise take
-// 129 VGPRs and 3 waves; the few registers spilled for it cost less than the
-// waves gained (clutter room: LT -2 %, BPT -3.6 % with the eye pass below).
+// The whole bounce with its rays traced here; true when the path has ended.
+template <bool WIDE, int MODE>
+__device__ __forceinline__ bool lt_bounce(const DrawParams& p, const TraceCtx& c, LtPath& s,
+                                          LightCacheEntryDev* __restrict__ staging) {
+  if (s.bounce >= p.maxPathLength) return true;
+  const ClosestHit h = trace_closest<WIDE>(c, s.o, s.d);
+  bool splats;
+  CameraSplat splat;
+  const bool goesOn = lt_shade<MODE>(p, s, h, staging, splats, splat);
+  if (splats && !trace_any<WIDE>(c, splat.o, splat.d, splat.tmax)) add_splat(p, splat.pixel, splat.color);
+  return !goesOn;
+}
+
+// The light paths as items of phased_paths.
+template <int MODE>
+struct LtProgram {
+  const DrawParams& p;
+  int raysPerSample;
+  LightCacheEntryDev *cache, *staging;
+  uint32_t* pathCounts;
+  gg::V3 o, d, lo, ld;
+  float ltmax;
+  gg::V3 tp, color;
+  uint32_t seed, gid, stored, pixel;
+  int bounce;
+  bool goesOn;
+
+  __device__ PathNext begin(uint32_t item) {
+    LtPath s;
+    lt_begin<MODE>(p, s, item, raysPerSample, cache);
+    take(s);
+    return p.maxPathLength > 0 ? kPathCloses : kPathEnds;
+  }
+  __device__ PathNext shade(int slot, float t, float by, float bz) {
+    LtPath s{tp, o, d, seed, gid, stored, bounce};
+    bool splats;
+    CameraSplat splat;
+    goesOn = lt_shade<MODE>(p, s, closest_from_record(p, slot, t, by, bz), staging, splats, splat);
+    take(s);
+    if (splats) {
+      lo = splat.o;
+      ld = splat.d;
+      ltmax = splat.tmax;
+      color = splat.color;
+      pixel = splat.pixel;
+      return kPathOccludes;
+    }
+    return goesOn ? kPathCloses : kPathEnds;
+  }
+  __device__ PathNext resolve(bool blocked) {
+    if (!blocked) add_splat(p, pixel, color);
+    return goesOn ? kPathCloses : kPathEnds;
+  }
+  __device__ void finish() {
+    if (MODE != kModeLT) pathCounts[gid] = stored;
+  }
+  __device__ void take(const LtPath& s) {
+    tp = s.tp;
+    o = s.o;
+    d = s.d;
+    seed = s.seed;
+    gid = s.gid;
+    stored = s.stored;
+    bounce = s.bounce;
+  }
+};
+
+// All numPaths light paths with path regeneration: over the reference layout, and
+// over the wide BVH where the paths stay in step (PathsInStep).  Five waves per
+// SIMD (at most 96 VGPRs).
 template <bool WIDE, int MODE>
 __global__ __launch_bounds__(kLightBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_lighttracer(
     DrawParams p, int raysPerSample, uint32_t numPaths, LightCacheEntryDev* __restrict__ cache,
-    LightCacheEntryDev* __restrict__ staging, uint32_t* __restrict__ pathCounts, uint32_t* __restrict__ queue) {
+    LightCacheEntryDev* __restrict__ staging, uint32_t* __restrict__ pathCounts, uint32_t* __restrict__ queue,
+    uint32_t /*lanes*/) {
   __shared__ uint2 stk[WIDE ? kWideLdsStack * kLightBlock : 1];
   const int tid = threadIdx.x;
   const uint32_t linear = blockIdx.x * kLightBlock + tid;
@@ -206,6 +287,23 @@ __global__ __launch_bounds__(kLightBlock) __attribute__((amdgpu_waves_per_eu(5))
       [&]() {
         if (MODE != kModeLT) pathCounts[s.gid] = s.stored;
       });
+}
+
+// The same over the wide BVH, in phases (phased_paths).  Room of 4000 spheres,
+// 1920x1080, path length 8: a light-traced frame 5.21 -> 3.86 ms.  Resident blocks
+// that take new paths (a block per 64 paths: 4.04 ms); four waves per SIMD (five:
+// 3.89 ms).
+template <int MODE, bool WT>
+__global__ __launch_bounds__(kLightBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_lighttracer_wide(
+    DrawParams p, int raysPerSample, uint32_t numPaths, LightCacheEntryDev* __restrict__ cache,
+    LightCacheEntryDev* __restrict__ staging, uint32_t* __restrict__ pathCounts, uint32_t* __restrict__ queue,
+    uint32_t lanes) {
+  __shared__ uint2 stk[kWideLdsStack * kLightBlock];
+  const uint32_t linear = blockIdx.x * kLightBlock + threadIdx.x;
+  LtProgram<MODE> prog{p, raysPerSample, cache, staging, pathCounts};
+  QueueChunks source{queue, (numPaths + lanes - 1u) / lanes};
+  phased_paths<WT, kWideLdsStack>(p.wide, stk, p.wide.spill + (size_t)linear * p.wide.spillDepth, numPaths, source,
+                                  lanes, prog);
 }
 
 // showlightcaches.comp:9-65 for exactly N light samples.
@@ -289,13 +387,74 @@ __device__ __forceinline__ bool bpt_eye_bounce(const DrawParams& p, const TraceC
   return bpt_eye_continue(p, s, v);
 }
 
+// The eye paths as items of phased_paths: the pixels of all 8x8 tiles.
+struct BptEyeProgram {
+  const DrawParams& p;
+  const LightCacheEntryDev* cache;
+  uint32_t actualN;
+  gg::V3 o, d, lo, ld;
+  float ltmax;
+  gg::V3 color, tp, add;
+  uint32_t seed, pixel;
+  int bounce;
+  float lastConnectionProbability, lastCosAbs;
+  bool goesOn;
+
+  __device__ PathNext begin(uint32_t item) {
+    int gx, gy;
+    tile_pixel(item, p.width, gx, gy);
+    BptEyePath s;
+    bpt_eye_begin(p, s, gx, gy);
+    pixel = (uint32_t)gy * (uint32_t)p.width + (uint32_t)gx;
+    take(s);
+    return p.maxPathLength > 0 ? kPathCloses : kPathEnds;
+  }
+  __device__ PathNext shade(int slot, float t, float by, float bz) {
+    if (slot < 0) return kPathEnds;
+    BptEyePath s{color, tp, o, d, seed, bounce, lastConnectionProbability, lastCosAbs, 0.0f};
+    BptEyeVertex v;
+    bpt_eye_hit(p, s, closest_from_record(p, slot, t, by, bz), v);
+    const BptConnection cn = bpt_connect_setup(p, s, cache, actualN);
+    bool occludes = false;
+    if (cn.test) {  // the value first: a zero one needs no ray (bpt_value_is_zero)
+      add = bpt_connect_value(p, s, v, cn, (float)actualN);
+      occludes = !bpt_value_is_zero(add);
+      lo = cn.lo;
+      ld = cn.ld;
+      ltmax = cn.tmax;
+    }
+    goesOn = !bpt_eye_continue(p, s, v);
+    take(s);
+    return occludes ? kPathOccludes : goesOn ? kPathCloses : kPathEnds;
+  }
+  __device__ PathNext resolve(bool blocked) {
+    if (!blocked) color = color + add;
+    return goesOn ? kPathCloses : kPathEnds;
+  }
+  __device__ void finish() {
+    float4* px = &p.accum[pixel];
+    const float4 v = *px;
+    *px = make_float4(color.x + v.x, color.y + v.y, color.z + v.z, 1.0f + v.w);
+  }
+  __device__ void take(const BptEyePath& s) {
+    color = s.color;
+    tp = s.tp;
+    o = s.o;
+    d = s.d;
+    seed = s.seed;
+    bounce = s.bounce;
+    lastConnectionProbability = s.lastConnectionProbability;
+    lastCosAbs = s.lastCosAbs;
+  }
+};
+
 // Eye paths of all pixels of the 8x8 tiles with path regeneration
-// (persistent_items); each pixel is written by one lane.
+// (persistent_items); each pixel is written by one lane.  Over the reference
+// layout, and over the wide BVH where the paths stay in step (PathsInStep).
 template <bool WIDE>
-// Five waves per SIMD, as k_lighttracer.
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_bpt_eye(DrawParams p, const LightCacheEntryDev* __restrict__ cache,
-                                                          const uint32_t* __restrict__ numEntriesPtr,
-                                                          uint32_t* __restrict__ queue) {
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_bpt_eye(
+    DrawParams p, const LightCacheEntryDev* __restrict__ cache, const uint32_t* __restrict__ numEntriesPtr,
+    uint32_t* __restrict__ queue, uint32_t /*lanes*/) {
   __shared__ uint2 stk[WIDE ? kWideLdsStack * kTileThreads : 1];
   const int tid = threadIdx.x;
   const uint32_t linear = blockIdx.x * kTileThreads + tid;
@@ -319,9 +478,31 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(5)
       });
 }
 
+// The same over the wide BVH, in phases (phased_paths).  Room of 4000 spheres,
+// 1920x1080, path length 8: a bidirectional frame, light pass included, 15.9 ->
+// 12.0 ms.  Four waves per SIMD with 80 bytes a lane spilled in the shading; three
+// without take 12.8 ms.
+template <bool WT>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_bpt_eye_wide(
+    DrawParams p, const LightCacheEntryDev* __restrict__ cache, const uint32_t* __restrict__ numEntriesPtr,
+    uint32_t* __restrict__ queue, uint32_t lanes) {
+  __shared__ uint2 stk[kWideLdsStack * kTileThreads];
+  const uint32_t linear = blockIdx.x * kTileThreads + threadIdx.x;
+  const int numEntries = (int)*numEntriesPtr;
+  const uint32_t pixels = ((uint32_t)p.width / kTile) * ((uint32_t)p.height / kTile) * kTileThreads;
+  BptEyeProgram prog{p, cache, (uint32_t)(numEntries < p.bptCapacity ? numEntries : p.bptCapacity)};
+  QueueChunks source{queue, (pixels + lanes - 1u) / lanes};
+  phased_paths<WT, kWideLdsStack>(p.wide, stk, p.wide.spill + (size_t)linear * p.wide.spillDepth, pixels, source,
+                                  lanes, prog);
+}
+
 // ---------------------------------------------------------------------------
+// Spill slices for `threads` lanes, and for every lane of a grid of blocks that
+// carry fewer than 64 items each (at most one block per SIMD).
 static hipError_t PrepareSpill(IntegratorState* st, DrawParams* p, size_t threads) {
   if (!p->useWide) return hipSuccess;
+  if (hipError_t e = EnsureSimds(st)) return e;
+  threads = std::max(threads, (size_t)st->simds * kTileThreads);
   const size_t bytes = std::max<size_t>(8, threads * p->wide.spillDepth * sizeof(uint2));
   hipError_t e = EnsureBuffer(&st->spill, &st->spillBytes, bytes);
   if (e == hipSuccess) p->wide.spill = (uint2*)st->spill;
@@ -329,23 +510,25 @@ static hipError_t PrepareSpill(IntegratorState* st, DrawParams* p, size_t thread
 }
 
 // The light paths of whole 64-path work groups (the reference dispatches
-// numPaths / 64 groups), one block per group.
+// numPaths / 64 groups): in phases by the resident blocks, else one block per group.
 template <int MODE>
 static hipError_t LaunchLight(IntegratorState* st, const DrawParams& p, int R, uint32_t numPaths,
                               LightCacheEntryDev* cache, LightCacheEntryDev* staging, uint32_t* counts,
                               hipStream_t stream) {
   const uint32_t paths = numPaths / kLightBlock * kLightBlock;
   if (paths == 0) return hipSuccess;
-  const void* fn = p.useWide ? reinterpret_cast<const void*>(&k_lighttracer<true, MODE>)
-                             : reinterpret_cast<const void*>(&k_lighttracer<false, MODE>);
-  uint32_t blocks = 0;
-  if (hipError_t e = PersistentGrid(st, fn, paths, &blocks, stream, false)) return e;
-  if (p.useWide)
-    hipLaunchKernelGGL((k_lighttracer<true, MODE>), dim3(blocks), dim3(kLightBlock), 0, stream, p, R, paths, cache,
-                       staging, counts, st->queue);
-  else
-    hipLaunchKernelGGL((k_lighttracer<false, MODE>), dim3(blocks), dim3(kLightBlock), 0, stream, p, R, paths, cache,
-                       staging, counts, st->queue);
+  typedef void (*Kernel)(DrawParams, int, uint32_t, LightCacheEntryDev*, LightCacheEntryDev*, uint32_t*, uint32_t*,
+                         uint32_t);
+  if (hipError_t e = EnsureSimds(st)) return e;
+  const bool phased = p.useWide && !PathsInStep(st, p, paths);
+  const Kernel fn = phased ? (p.watertight ? k_lighttracer_wide<MODE, true> : k_lighttracer_wide<MODE, false>)
+                           : (p.useWide ? k_lighttracer<true, MODE> : k_lighttracer<false, MODE>);
+  uint32_t blocks = 0, lanes = kLightBlock;
+  if (hipError_t e = PersistentGrid(st, reinterpret_cast<const void*>(fn), paths, &blocks, stream, phased,
+                                    phased ? &lanes : nullptr))
+    return e;
+  hipLaunchKernelGGL(fn, dim3(blocks), dim3(kLightBlock), 0, stream, p, R, paths, cache, staging, counts, st->queue,
+                     lanes);
   return hipGetLastError();
 }
 
@@ -440,14 +623,15 @@ hipError_t DrawBPT(IntegratorState* st, const DrawParams& p0, hipStream_t stream
   if (e != hipSuccess || !err->empty()) return e;
   const size_t pixels = (size_t)(p.width / kTile) * (p.height / kTile) * kTileThreads;
   if (pixels) {
-    const void* fn = p.useWide ? reinterpret_cast<const void*>(&k_bpt_eye<true>)
-                               : reinterpret_cast<const void*>(&k_bpt_eye<false>);
-    uint32_t blocks = 0;
-    if (hipError_t e2 = PersistentGrid(st, fn, pixels, &blocks, stream)) return e2;
-    if (p.useWide)
-      hipLaunchKernelGGL(k_bpt_eye<true>, dim3(blocks), dim3(kTileThreads), 0, stream, p, cache, total, st->queue);
-    else
-      hipLaunchKernelGGL(k_bpt_eye<false>, dim3(blocks), dim3(kTileThreads), 0, stream, p, cache, total, st->queue);
+    typedef void (*Kernel)(DrawParams, const LightCacheEntryDev*, const uint32_t*, uint32_t*, uint32_t);
+    const bool phased = p.useWide && !PathsInStep(st, p, pixels);
+    const Kernel fn = phased ? (p.watertight ? k_bpt_eye_wide<true> : k_bpt_eye_wide<false>)
+                             : (p.useWide ? k_bpt_eye<true> : k_bpt_eye<false>);
+    uint32_t blocks = 0, lanes = kTileThreads;
+    if (hipError_t e2 = PersistentGrid(st, reinterpret_cast<const void*>(fn), pixels, &blocks, stream, true,
+                                       phased ? &lanes : nullptr))
+      return e2;
+    hipLaunchKernelGGL(fn, dim3(blocks), dim3(kTileThreads), 0, stream, p, cache, total, st->queue, lanes);
   }
   return hipGetLastError();
 }
