@@ -4,6 +4,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <new>
 #include <set>
 #include <string>
@@ -52,6 +53,7 @@ struct gpugi_ctx {
   void* dWideQueue = nullptr;  // the wide trace kernel's batch counters
   size_t spillBytes = 0;
   uint32_t wideMaxStack = 0, wideMaxPending = 0, wideNumNodes = 0;
+  std::map<int, int> wideBlocksPerCU;  // per LDS stack depth: resident blocks of the trace kernel
   int wideLeaf = 2;     // triangles per merged wide leaf
   int wideStack = 10;   // LDS stack entries per lane of the trace kernel
   int wideRefill = 8;   // idle lanes that trigger a wave-level ray refill
@@ -214,11 +216,21 @@ int EnsureSideStream(gpugi_ctx* ctx) {
   return GPUGI_OK;
 }
 
+// Resident blocks per CU of the trace kernel variant `stack` (asked for once).
+int ResidentBlocks(gpugi_ctx* ctx, int stack, int* blocks) {
+  int& known = ctx->wideBlocksPerCU[stack];
+  if (known == 0) {
+    HIP_TRY(ctx, WideBlocksPerCU(stack, &known));
+    if (known < 1) known = 1;
+  }
+  *blocks = known;
+  return GPUGI_OK;
+}
+
 // Persistent grid and spill buffer for the trace kernel variant `stack`.
 int PrepareTraceWide(gpugi_ctx* ctx, int stack, WideScene* out) {
   int blocksPerCU = 0;
-  HIP_TRY(ctx, WideBlocksPerCU(stack, &blocksPerCU));
-  if (blocksPerCU < 1) blocksPerCU = 1;
+  if (int rc = ResidentBlocks(ctx, stack, &blocksPerCU)) return rc;
   WideScene s = MakeWide(ctx, stack);
   // whole blocks per XCD for the static schedule of the trace kernel
   const uint32_t blocks = std::max<uint32_t>(8, (uint32_t)(ctx->numCUs * blocksPerCU) / 8 * 8);
@@ -1135,9 +1147,9 @@ int gpugi_trace(gpugi_ctx* ctx, int query, int kernel, const gpugi_ray* rays, gp
   if (n > 0xffffff00ull) return Fail(ctx, GPUGI_ERR_ARG, "gpugi_trace: at most 2^32 - 256 rays per call");
   if (n == 0) return GPUGI_OK;
   if (SetDev(ctx)) return GPUGI_ERR_HIP;
-  // the stack-overflow flag reports this call only (a fill kernel, so the call can be captured)
-  HIP_TRY(ctx, LaunchFillU32((uint32_t*)ctx->dCounters + 1, 0u, 1, ctx->stream));
   const bool wide = kernel == GPUGI_KERNEL_WIDE || (kernel == GPUGI_KERNEL_AUTO && ctx->hasWide);
+  // the stack-overflow flag, which only a call with host buffers reads, reports this call only
+  if (!rays_on_device) HIP_TRY(ctx, LaunchFillU32((uint32_t*)ctx->dCounters + 1, 0u, 1, ctx->stream));
   // pinned host buffers: chunked copies that overlap the traversal; pageable
   // ones go through one staged copy each way, which the runtime does faster
   if (!rays_on_device && n > ((size_t)1 << 22) && IsPinned(rays, n * sizeof(gpugi_ray)) &&
@@ -1180,7 +1192,6 @@ int gpugi_trace_noalloc(gpugi_ctx* ctx, int query, int kernel, const gpugi_ray* 
   if (n == 0) return GPUGI_OK;
   if (!ctx->noAllocScratch) return Fail(ctx, GPUGI_ERR_STATE, "gpugi_trace_noalloc: scratch not set up");
   if (SetDev(ctx)) return GPUGI_ERR_HIP;
-  HIP_TRY(ctx, LaunchFillU32((uint32_t*)ctx->dCounters + 1, 0u, 1, ctx->stream));
   const bool wide = kernel == GPUGI_KERNEL_WIDE || (kernel == GPUGI_KERNEL_AUTO && ctx->hasWide);
   if (!wide) {  // the escape walk keeps no stack: nothing but the caller's buffers
     HIP_TRY(ctx, LaunchTraceRef(MakeRef(ctx), query, rays, hits, n, Watertight(ctx), ctx->stream));
@@ -1188,8 +1199,7 @@ int gpugi_trace_noalloc(gpugi_ctx* ctx, int query, int kernel, const gpugi_ray* 
   }
   if (!ctx->hasWide) return Fail(ctx, GPUGI_ERR_STATE, "gpugi_trace_noalloc: no wide hierarchy");
   int blocksPerCU = 0;
-  HIP_TRY(ctx, WideBlocksPerCU(ctx->wideStack, &blocksPerCU));
-  if (blocksPerCU < 1) blocksPerCU = 1;
+  if (int rc = ResidentBlocks(ctx, ctx->wideStack, &blocksPerCU)) return rc;
   WideScene s = MakeWide(ctx, ctx->wideStack);
   // the resident grid (whole blocks per XCD), shrunk until its spill stacks fit the array
   uint32_t blocks = std::max<uint32_t>(8, (uint32_t)(ctx->numCUs * blocksPerCU) / 8 * 8);

@@ -4,7 +4,11 @@
 // b runs on XCD b % 8; XCD x owns the x-th contiguous eighth of the ray array
 // (neighbouring rays start close together, so they share that XCD's L2), and
 // its waves take that range's 64-ray batches in order from one atomic counter
-// per XCD, so no wave sits idle while its XCD has batches left.
+// per XCD, so no wave sits idle while its XCD has batches left.  A launch with a
+// wave for every batch takes no counters (s.queue null): wave w of an XCD has
+// batch w, and the kernel that zeroes the counters is not launched (257 rays in the
+// Cornell room 23 -> 17 us a call, 2^17 diffuse rays in the room of 4000 spheres
+// 263 -> 245 us, 2^18 295 -> 262).
 //
 // Each wave runs its 64 lanes one box or leaf pass at a time (trace_wide.h);
 // a leaf pass is chosen when at least `wait` lanes have only a pending leaf.
@@ -39,6 +43,19 @@ __global__ void k_wide_queue_reset(uint32_t* q) {
   if (threadIdx.x < (unsigned)kWideQueueWords) q[threadIdx.x] = 0u;
 }
 
+// The launch of n rays: the persistent grid of s.numThreads, or fewer blocks (whole
+// blocks per XCD) when those give every 64-ray batch a wave.
+struct WideGrid {
+  uint32_t blocks;
+  bool counters;
+};
+WideGrid GridFor(const WideScene& s, size_t n) {
+  constexpr size_t kWaves = kWideBlock / 64;
+  const size_t batches = (n + 63) / 64, perXcd = (batches + kNumXcd - 1) / kNumXcd;
+  const size_t need = (perXcd + kWaves - 1) / kWaves * kNumXcd, most = s.numThreads / kWideBlock;
+  return need <= most ? WideGrid{(uint32_t)need, false} : WideGrid{(uint32_t)most, true};
+}
+
 template <bool ANY, int B, int S, bool WT>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_trace_wide(WideScene s, const float4* __restrict__ rays,
                                                   int4* __restrict__ hits, uint32_t n, int refill, int wait,
@@ -48,7 +65,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_t
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const uint32_t gtid = blockIdx.x * B + tid;
-  // spill laid out [depth][thread] over the whole grid (s.numThreads == gridDim.x * B)
+  // spill laid out [depth][thread] over the whole grid (gridDim.x * B <= s.numThreads)
   const WideStack stk{as_lds(lds), tid, s.spill + gtid, gridDim.x * (uint32_t)B};
 
   const uint32_t xcd = blockIdx.x % kNumXcd;
@@ -59,8 +76,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_t
   uint32_t* counter = s.queue + xcd * kWideQueueStride;
   const uint64_t below = (1ull << lane) - 1ull;
 
-  // wave-uniform: the batch being handed out and how many of its rays are gone
+  // wave-uniform: the batch being handed out and how many of its rays are gone,
+  // and the wave's batch where there are no counters
   uint32_t curBatch = 0, curPos = 64;
+  uint32_t ownBatch = blockIdx.x / kNumXcd * (B / 64u) + (uint32_t)__builtin_amdgcn_readfirstlane(tid / 64);
   bool exhausted = bBegin >= bEnd;
   bool active = false;
   uint32_t ri = 0;
@@ -73,9 +92,13 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_t
       const uint32_t avail = 64u - curPos;
       uint32_t next = bEnd;
       if (avail < nidle) {  // take the XCD's next batch
-        uint32_t v = 0;
-        if (lane == 0) v = atomicAdd(counter, 1u);
-        v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+        uint32_t v = ownBatch;
+        if (s.queue) {
+          if (lane == 0) v = atomicAdd(counter, 1u);
+          v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+        } else {
+          ownBatch = batches;  // taken
+        }
         if (v < bEnd - bBegin) next = bBegin + v;
       }
       if (!active) {
@@ -136,9 +159,12 @@ const Variant* FindVariant(int stack) {
 }
 
 template <int S, bool WT>
-void LaunchS(const WideScene& s, int query, const gpugi_ray* rays, gpugi_hit* hits, size_t n, int refill,
+void LaunchS(const WideScene& scene, int query, const gpugi_ray* rays, gpugi_hit* hits, size_t n, int refill,
              int wait, hipStream_t stream, const uint32_t* nDev) {
-  dim3 grid(s.numThreads / kWideBlock);
+  const WideGrid g = GridFor(scene, n);
+  WideScene s = scene;
+  if (!g.counters) s.queue = nullptr;
+  dim3 grid(g.blocks);
   if (query == GPUGI_ANY_HIT)
     hipLaunchKernelGGL((k_trace_wide<true, kWideBlock, S, WT>), grid, dim3(kWideBlock), 0, stream, s,
                        (const float4*)rays, (int4*)hits, (uint32_t)n, refill, wait, nDev);
@@ -179,7 +205,8 @@ hipError_t LaunchTraceWide(const WideScene& s, int stack, int query, const gpugi
   if (s.numThreads == 0 || s.numThreads % (kWideBlock * kNumXcd) != 0) return hipErrorInvalidConfiguration;
   if (refill < 1 || refill > 64 || wait < 1 || wait > 64) return hipErrorInvalidValue;
   if (!s.queue) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_wide_queue_reset, dim3(1), dim3(kWideQueueWords), 0, stream, s.queue);
+  if (GridFor(s, n).counters)
+    hipLaunchKernelGGL(k_wide_queue_reset, dim3(1), dim3(kWideQueueWords), 0, stream, s.queue);
   switch (stack) {
     case 4: LaunchS<4>(s, query, rays, hits, n, refill, wait, watertight, stream, nDevice); break;
     case 8: LaunchS<8>(s, query, rays, hits, n, refill, wait, watertight, stream, nDevice); break;
