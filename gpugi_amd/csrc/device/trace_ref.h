@@ -266,4 +266,84 @@ __device__ __forceinline__ bool trace_ref(const RefScene& s, gg::V3 o, gg::V3 d,
   return false;
 }
 
+// The same walk one step at a time, for kernels that run the lanes of a wave
+// through box and triangle steps together (k_trace_ref): per ray the same
+// operations on the same values in the same order as trace_ref without the
+// importance break, so the same result.
+struct RefWalk {
+  gg::V3 o, d, inv;
+  float t;          // rayLength
+  int node;         // next node to test (0 after the first step: none)
+  int leaf;         // next triangle slot to test, -1: none
+  int slot;         // the hit's slot, -1: none
+  float by, bz;     // its barycentrics
+  bool found;       // ANY
+  WtRay wr;         // watertight test only
+};
+
+template <bool WT>
+__device__ __forceinline__ void ref_walk_init(RefWalk& w, gg::V3 o, gg::V3 d, float tmax) {
+  w.o = o;
+  w.d = d;
+  w.inv = gg::v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+  w.t = tmax;
+  w.node = 0;
+  w.leaf = -1;
+  w.slot = -1;
+  w.by = w.bz = 0.0f;
+  w.found = false;
+  if (WT) w.wr = wt_setup(d);
+}
+
+// For a ray without a leaf to test: tests its next node.  True when the walk has ended.
+template <bool OBOX>
+__device__ __forceinline__ bool ref_walk_box(const RefScene& s, RefWalk& w) {
+  float newHit, exitDist;
+  bool boxHit;
+  float4 a, b;
+  if (OBOX) {
+    a = s.nodes[3 * w.node];
+    b = s.nodes[3 * w.node + 1];
+    boxHit = intersect_obox(w.o, w.d, a, b, s.nodes[3 * w.node + 2], newHit, exitDist);
+  } else {
+    a = s.nodes[2 * w.node];
+    b = s.nodes[2 * w.node + 1];
+    boxHit = intersect_box(w.o, w.inv, gg::v3(a.x, a.y, a.z), gg::v3(b.x, b.y, b.z), newHit, exitDist);
+  }
+  const uint32_t childCode = __float_as_uint(a.w);
+  const int escape = __float_as_int(b.w), child = (int)(childCode & 0x7fffffffu);
+  const bool enters = boxHit && newHit <= w.t, isLeaf = (childCode & 0x80000000u) != 0u;
+  w.leaf = enters && isLeaf ? 2 * child : -1;
+  w.node = enters && !isLeaf ? child : escape;
+  return w.node == 0 && w.leaf < 0;
+}
+
+// For a ray with a leaf to test: tests its triangles.  True when the walk has ended.
+template <bool ANY, bool WT>
+__device__ __forceinline__ bool ref_walk_leaf(const RefScene& s, RefWalk& w) {
+  for (int leaf = w.leaf;;) {
+    const int4 tri = s.slots[leaf];
+    if (tri.x == tri.y) break;
+    const gg::V3 p0 = load_pos(s.positions, tri.x), p1 = load_pos(s.positions, tri.y), p2 = load_pos(s.positions, tri.z);
+    float newHit;
+    gg::V3 bary, n;
+    const bool ok = WT ? intersect_triangle_wt(w.o, w.wr, p0, p1, p2, newHit, bary)
+                       : intersect_triangle(w.o, w.d, p0, p1, p2, newHit, bary, n);
+    if (ok && newHit < w.t) {
+      if (ANY) {
+        w.found = true;
+        return true;
+      }
+      w.t = newHit;
+      w.slot = leaf;
+      w.by = bary.y;
+      w.bz = bary.z;
+    }
+    ++leaf;
+    if (leaf % 2 == 0) break;
+  }
+  w.leaf = -1;
+  return w.node == 0;
+}
+
 }  // namespace gpugi

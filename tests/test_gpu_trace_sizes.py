@@ -28,17 +28,19 @@ def ray_set(rt):
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 512, 513, 2049, RESIDENT - 64, RESIDENT, RESIDENT + 1, MOST])
 @pytest.mark.parametrize("query", ["closest", "any"])
-def test_prefixes_of_a_ray_set(rt, ray_set, query, n):
+@pytest.mark.parametrize("kernel", ["wide", "reference"])
+def test_prefixes_of_a_ray_set(rt, ray_set, kernel, query, n):
     c, sets = ray_set
-    print("case: %s, %d rays" % (query, n), flush=True)
+    print("case: %s, %s, %d rays" % (kernel, query, n), flush=True)
     rays, q = (sets.incoherent, rt.CLOSEST_HIT) if query == "closest" else (sets.shadow, rt.ANY_HIT)
     cols = slice(0, 4) if query == "closest" else slice(0, 1)
     c.trace_device(rays, sets.hits, MOST, q, rt.KERNEL_REFERENCE)
     want = sets.hits.download(np.int32, 4 * MOST).reshape(-1, 4)
     mark = np.full((MOST, 4), -77, np.int32)
     sets.hits.upload(mark)
-    c.trace_device(rays, sets.hits, n, q, rt.KERNEL_WIDE)
+    c.trace_device(rays, sets.hits, n, q, rt.KERNEL_WIDE if kernel == "wide" else rt.KERNEL_REFERENCE)
     got = sets.hits.download(np.int32, 4 * MOST).reshape(-1, 4)
     assert (got[n:] == -77).all()
-    # an edge or a tie may differ from the reference walk: none does on these sets' first rays
-    assert (got[:n, cols] != want[:n, cols]).any(1).sum() <= n // 100000
+    # an edge or a tie may differ between the walks
+    most = n // 100000 if kernel == "wide" else 0
+    assert (got[:n, cols] != want[:n, cols]).any(1).sum() <= most
