@@ -70,6 +70,40 @@ def test_importance_and_materials_match_oracle(rt, oracle, ctx, name, bvh):
         ctx.set_bvh_type(rt.BVH_AABOX)
 
 
+@pytest.mark.parametrize("bvh", ["aabox", "obox"])
+@pytest.mark.parametrize("cells", [1, 2, 3])
+def test_importance_on_small_trees_matches_oracle(rt, oracle, ctx, cells, bvh):
+    """Trees of one to a few levels (walks that enter all, some or none of a
+    node's children), bit for bit: the sums are exact (32 x 32 paths)."""
+    print("case: hierarchy small %d %s" % (cells, bvh), flush=True)
+    hs = rt.HostScene.heightfield(cells, workloads.MASTER_SEED)
+    for p in workloads.heightfield_lights():
+        hs.add_point_light(p, (0.5, 0.5, 0.5))
+    ctx.set_bvh_type(rt.BVH_OBOX if bvh == "obox" else rt.BVH_AABOX)
+    try:
+        ctx.load_scene(hs)
+        arrays = hs.arrays()
+        if bvh == "obox":
+            arrays["obox"] = hs.obox_hierarchy()
+        sc = oracle.Scene(arrays)
+        w = h = 32
+        cam = workloads.heightfield_camera(w, h)
+        ctx.set_screen(w, h)
+        ctx.set_camera(cam)
+        ls = rt.LightSampler(hs, 3).generate(64)
+        ctx.set_light_samples(ls)
+        ctx.hierarchy_update_importance(4)
+        imp, sub = ctx.hierarchy_read()
+        want = np.zeros((len(sc.a["hierarchy"]) + len(sc.a["triangles"]), 2), np.float32)
+        for it in range(1, 5):
+            oracle.hier_acquire(sc, ls, cam, w, h, it, want)
+        want, want_sub = oracle.hier_propagate(sc, 4, want)
+        assert want[0, 0] > 0
+        assert same(imp, want) and same(sub, want_sub)
+    finally:
+        ctx.set_bvh_type(rt.BVH_AABOX)
+
+
 def test_hierarchy_state_errors(rt, ctx):
     ctx.load_scene(rt.HostScene.cornell())
     with pytest.raises(rt.GpugiError):
