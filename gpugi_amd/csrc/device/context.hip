@@ -545,7 +545,7 @@ int gpugi_set_pt_schedule(gpugi_ctx* ctx, int schedule) {
 namespace {
 
 size_t Align256(size_t b) { return (b + 255) & ~(size_t)255; }
-int MlpEnsureTiles(gpugi_ctx* ctx, uint32_t tiles);
+int MlpEnsureParts(gpugi_ctx* ctx, size_t n);
 
 // Scene bounds as the cache's position mapping: min and 1 / extent per axis.
 int SceneBounds(gpugi_ctx* ctx, float mn[3], float invExtent[3]) {
@@ -667,7 +667,7 @@ int DrawCached(gpugi_ctx* ctx, uint32_t frameSeed) {
   ctx->dCacheCount = dTotal;
   const int steps = ctx->cacheTrainSteps;
   if (steps > 0) {
-    if (int rc = MlpEnsureTiles(ctx, MlpTiles(S / (uint32_t)steps))) return rc;
+    if (int rc = MlpEnsureParts(ctx, S / (uint32_t)steps)) return rc;
     for (int s = 0; s < steps; ++s) {
       const MlpBatch batch{dTotal, S, (uint32_t)s, (uint32_t)steps};
       HIP_TRY(ctx, LaunchMlpGradientTiles(ctx->mlp, feat, targets, batch, trainStream));
@@ -1626,14 +1626,16 @@ void MlpInitialWeights(uint64_t seed, std::vector<float>* w) {
   }
 }
 
-int MlpEnsureTiles(gpugi_ctx* ctx, uint32_t tiles) {
-  if (ctx->mlp.partialTiles >= tiles) return GPUGI_OK;
+// Partials for gradient steps of at most n samples.
+int MlpEnsureParts(gpugi_ctx* ctx, size_t n) {
+  const uint32_t parts = MlpParts((uint32_t)std::min<size_t>(n, 0xffffffffu), MlpGradTileLog2(n));
+  if (ctx->mlp.partialBlocks >= parts) return GPUGI_OK;
   FreeDev(*(void**)&ctx->mlp.partials);
   FreeDev(*(void**)&ctx->mlp.loss);
-  ctx->mlp.partialTiles = 0;
-  HIP_TRY(ctx, hipMalloc((void**)&ctx->mlp.partials, (size_t)tiles * kMlpParams * sizeof(float)));
-  HIP_TRY(ctx, hipMalloc((void**)&ctx->mlp.loss, (size_t)tiles * sizeof(float)));
-  ctx->mlp.partialTiles = tiles;
+  ctx->mlp.partialBlocks = 0;
+  HIP_TRY(ctx, hipMalloc((void**)&ctx->mlp.partials, (size_t)parts * kMlpParams * sizeof(float)));
+  HIP_TRY(ctx, hipMalloc((void**)&ctx->mlp.loss, (size_t)parts * sizeof(float)));
+  ctx->mlp.partialBlocks = parts;
   return GPUGI_OK;
 }
 
@@ -1748,7 +1750,7 @@ namespace {
 int MlpGradientCommon(gpugi_ctx* ctx, const char* fn, const float* features, const float* targets, size_t n,
                       int on_device, const AdamParams* adam = nullptr) {
   if (n == 0 || !features || !targets) return Fail(ctx, GPUGI_ERR_ARG, std::string(fn) + ": need samples");
-  if (int rc = MlpEnsureTiles(ctx, MlpTiles(n))) return rc;
+  if (int rc = MlpEnsureParts(ctx, n)) return rc;
   const float* df = features;
   const float* dt = targets;
   const size_t fb = n * kMlpRaw * sizeof(float), tb = n * 4 * sizeof(float);

@@ -62,14 +62,28 @@ struct MlpDev {
   uint16_t* wb;      // kMlpParams BF16 weights [out][in]
   uint16_t* wtb;     // kMlpWTSize BF16 transposed weights [in][out32]
   uint16_t* wbi;     // kMlpInferSize BF16 inference copy (padded rows, permuted columns)
-  float* partials;   // per-tile gradient partials (grad kernel)
-  uint32_t partialTiles;
+  float* partials;   // gradient partials, one per block of the grad kernel
+  uint32_t partialBlocks;
   float* grad;       // kMlpParams reduced gradient
-  float* loss;       // per-tile loss partials
+  float* loss;       // loss partials, likewise
 };
 
-// Tiles of 32 samples the gradient kernel processes.
-inline uint32_t MlpTiles(size_t n) { return (uint32_t)((n + 31) / 32); }
+// The gradient kernel's most blocks, so partials: one per CU.
+constexpr uint32_t kMlpGradBlocks = 256;
+// log2 of the samples in a tile of the gradient kernel, for steps of at most n
+// samples (which fixes the kernel, whatever a count on the device then says): 64
+// (eight waves) where the partials are what a step waits for, 32 (four waves)
+// where it is the chain of phases (16 steps and an inference: 0.351 -> 0.338 ms
+// for 257 samples a step, 0.427 -> 0.413 for 4,096, 0.621 -> 0.531 for 16,384; with
+// 64 below the line 0.367 for 257 and 0.372 for 1,000, which take 0.351 with 32).
+constexpr uint32_t kMlpGradSmall = 2048;
+inline uint32_t MlpGradTileLog2(size_t n) { return n <= kMlpGradSmall ? 5u : 6u; }
+static_assert(kMlpGradSmall <= 32 * kMlpGradBlocks, "the four-wave kernel has one tile per block");
+// The blocks, so partials, of n samples.
+__host__ __device__ inline uint32_t MlpParts(uint32_t n, uint32_t tileLog2) {
+  const uint32_t tiles = (n >> tileLog2) + ((n & ((1u << tileLog2) - 1u)) != 0u);
+  return tiles < kMlpGradBlocks ? tiles : kMlpGradBlocks;
+}
 
 // Samples of one training step.  With count == nullptr: samples [0, n).  With
 // a device counter: total = min(*count, n) samples are split into `steps`
@@ -100,8 +114,8 @@ hipError_t LaunchMlpInfer(const MlpDev& m, const float* raw, float* radiance, si
 // Gradient of the relative L2 loss mean_{s,c<3} (y - t)^2 / (y^2 + 0.01) (y treated as a
 // constant in the denominator) over the samples of `batch` into m.grad, and the loss
 // into *lossOut (device scalar); both are 0 for an empty batch.  raw / targets:
-// n x 16 / n x 4 floats.  Needs m.partialTiles >= MlpTiles(batch.n / batch.steps).
-// Two launches: the per-tile partial gradients, then their fixed-order sum.
+// n x 16 / n x 4 floats.  Needs m.partialBlocks >= MlpParts of batch.n / batch.steps.
+// Two launches: the partial gradients, then their fixed-order sum.
 hipError_t LaunchMlpGradient(const MlpDev& m, const float* raw, const float* targets, const MlpBatch& batch,
                              float* lossOut, hipStream_t stream);
 // The same two launches separately; with `adam` the sum also applies the Adam

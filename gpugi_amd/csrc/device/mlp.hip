@@ -8,10 +8,10 @@
 // so each lane reads 16 contiguous bytes of a weight row and of an activation
 // row (LDS, sample-major) per instruction and writes back 4 outputs of one
 // sample.  The backward pass uses the same instruction for
-//   dW_l = dY_l^T X_l      (K = the 32 samples of a tile; feature-major copies)
+//   dW_l = dY_l^T X_l      (K = the samples of a tile; feature-major copies)
 //   dX_l = W_l^T dY_l      (A = the transposed weights WT_l[in][out32])
-// Gradients are written per 32-sample tile (four waves per tile) and summed in
-// a fixed order (tile classes t mod 16 in tile order, then a pairwise tree over
+// A block sums the gradients of its tiles (t, t + 256, ...) in registers and
+// writes one partial; the partials are summed in a fixed order (classes t mod 16 in order, then a pairwise tree over
 // the classes), so a training step is deterministic; the Adam step runs in the
 // same launch as that sum.
 #include <hip/hip_runtime.h>
@@ -122,7 +122,6 @@ __device__ __forceinline__ void encode_part(const float* __restrict__ raw, int q
 
 constexpr int kActStride = 104;  // sample-major rows: 96 features + 8 pad (bf16 elements)
 constexpr int kHidStride = 72;   // 64 + 8
-constexpr int kSmpStride = 40;   // feature-major rows: 32 samples + 8
 
 // ---------------------------------------------------------------- inference
 //
@@ -367,29 +366,39 @@ __global__ __launch_bounds__(kInferBlock) void k_mlp_infer(const uint16_t* __res
 
 // ---------------------------------------------------------------- gradient
 
-// Four waves share one 32-sample tile; every phase splits its 16 x 16 output
-// blocks over the waves (each block is computed by one wave with the same
+// WAVES waves share one tile of 8 * WAVES samples; every phase splits its 16 x 16
+// output blocks over the waves (each block is computed by one wave with the same
 // instruction sequence whatever the split, so the split changes no bit).
-constexpr int kGradWaves = 4;
-constexpr int kGradBlock = 64 * kGradWaves;
-
+//
+// Bound by the memory traffic of the partials (78 KB each, written here and read by
+// k_mlp_reduce) and by the chain of ten phases.  Eight waves halve the partials,
+// and a block keeps its partial in registers over its tiles, so that there are
+// at most kMlpGradBlocks (20 MB) for any batch: 16 Adam steps and an inference of
+// 64 samples take 0.614 -> 0.531 ms for 16,384 samples a step and 1.42 -> 0.98 ms
+// for 65,536, against one partial per 32-sample tile (40 and 160 MB each way).
+// One block of eight waves per CU (138 KB of LDS).  Four waves (MlpGradTileLog2)
+// run one tile per block.
+template <int WAVES>
 struct GradLds {
-  uint16_t a0[32 * kActStride];            // encoded inputs, sample-major
-  uint16_t a[4][32 * kHidStride];          // hidden outputs 1..4, sample-major
+  static constexpr int kTile = 8 * WAVES;
+  static constexpr int kSmpStride = kTile + 8;  // feature-major rows
+  uint16_t a0[kTile * kActStride];    // encoded inputs, sample-major
+  uint16_t a[4][kTile * kHidStride];  // hidden outputs 1..4, sample-major
   uint16_t t0[kMlpIn * kSmpStride];        // encoded inputs, feature-major
   uint16_t t[4][kMlpHidden * kSmpStride];  // hidden outputs, feature-major
-  uint16_t dys[2][32 * kHidStride];        // dY, sample-major (ping-pong)
+  uint16_t dys[2][kTile * kHidStride];  // dY, sample-major (ping-pong)
   uint16_t dyt[2][kMlpHidden * kSmpStride];  // dY, feature-major
-  float loss[2];                           // the two halves' loss sums
+  float loss[4];                               // loss sums per 16 samples
 };
 
-// Forward of layer l for half h (samples 16h..16h+15) of the tile and output
+// Forward of layer l for group h (samples 16h..16h+15) of the tile and output
 // blocks ob0, ob0 + 1, K_IN inputs from the sample-major `src` rows; ReLU
 // outputs go to `dst` (sample-major) and `dstT` (feature-major).
-template <int K_IN>
+template <int WAVES, int K_IN>
 __device__ __forceinline__ void grad_fwd_hidden(const uint16_t* __restrict__ W, const uint16_t* src, int srcStride,
                                                 uint16_t* dst, uint16_t* dstT, int h, int ob0, int lane) {
   const int s = lane & 15, q = lane >> 4;
+  constexpr int kSmpStride = GradLds<WAVES>::kSmpStride;
   const int smp = 16 * h + s;
   f32x4 acc[2];
 #pragma unroll
@@ -413,33 +422,57 @@ __device__ __forceinline__ void grad_fwd_hidden(const uint16_t* __restrict__ W, 
   }
 }
 
-// dW_l (rows OUT_L, K_IN columns) += dY^T X over the tile's 32 samples: the
-// (ob, ib) blocks numbered ob * (K_IN / 16) + ib, block b on wave b mod 4.
-template <int OUT_L, int K_IN>
-__device__ __forceinline__ void grad_dw(const uint16_t* dyt, const uint16_t* xt, float* __restrict__ part, int wave,
-                                        int lane) {
+// 16 x 16 blocks of dW_l (OUT_L rows, K_IN columns) a wave has: those numbered
+// ob * (K_IN / 16) + ib are on wave number mod `waves`.
+constexpr int grad_dw_blocks(int waves, int out, int in) { return (out / 16 * (in / 16) + waves - 1) / waves; }
+
+// acc += the wave's blocks of dY^T X over the tile's samples; the last tile of the
+// block writes them to its partial, beside the phases that follow.
+template <int WAVES, int OUT_L, int K_IN>
+__device__ __forceinline__ void grad_dw(const uint16_t* dyt, const uint16_t* xt,
+                                        f32x4 (&acc)[grad_dw_blocks(WAVES, OUT_L, K_IN)], bool last,
+                                        float* __restrict__ part, int wave, int lane) {
   const int s = lane & 15, q = lane >> 4;
-  constexpr int kIb = K_IN / 16;
-#pragma unroll 2
-  for (int b = wave; b < (OUT_L / 16) * kIb; b += kGradWaves) {
-    const int ob = b / kIb, ib = b % kIb;
-    const f32x4 d = mfma(ld8(dyt + (16 * ob + s) * kSmpStride + 8 * q), ld8(xt + (16 * ib + s) * kSmpStride + 8 * q),
-                         f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+  constexpr int kSmpStride = GradLds<WAVES>::kSmpStride;
+  constexpr int kIb = K_IN / 16, kBlocks = OUT_L / 16 * kIb;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) part[(16 * ob + 4 * q + v) * K_IN + 16 * ib + s] = d[v];
+  for (int i = 0; i < grad_dw_blocks(WAVES, OUT_L, K_IN); ++i) {
+    const int b = wave + i * WAVES;
+    if (kBlocks % WAVES != 0 && b >= kBlocks) break;
+    const int ob = b / kIb, ib = b % kIb;
+    // products of 32 samples from zero and their sum, not one chain: the error is
+    // that of one partial per 32 samples (measured equal against FP64)
+    f32x4 d[WAVES / 4];
+#pragma unroll
+    for (int ks = 0; ks < WAVES / 4; ++ks)
+      d[ks] = mfma(ld8(dyt + (16 * ob + s) * kSmpStride + 32 * ks + 8 * q),
+                   ld8(xt + (16 * ib + s) * kSmpStride + 32 * ks + 8 * q), f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[i][v] += WAVES == 8 ? d[0][v] + d[WAVES / 4 - 1][v] : d[0][v];
+    if (last) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part[(16 * ob + 4 * q + v) * K_IN + 16 * ib + s] = acc[i][v];
+    }
   }
+}
+
+template <int N>
+__device__ __forceinline__ void grad_zero(f32x4 (&acc)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 }
 
 // dX_l = W_l^T dY_l (K = OUT32 outputs), gated by the ReLU of the layer input
 // x (sample-major, 64 features), into the next dY buffers: input block
-// ib = wave, both halves.
-template <int OUT32>
+// ib = wave mod 4, two groups of 16 samples.
+template <int WAVES, int OUT32>
 __device__ __forceinline__ void grad_dx(const uint16_t* __restrict__ WT, const uint16_t* dys, const uint16_t* x,
                                         uint16_t* ndys, uint16_t* ndyt, int wave, int lane) {
   const int s = lane & 15, q = lane >> 4;
-  const int ib = wave;
+  constexpr int kSmpStride = GradLds<WAVES>::kSmpStride;
+  const int ib = wave & 3, h0 = 2 * (wave >> 2);
 #pragma unroll 1
-  for (int h = 0; h < 2; ++h) {
+  for (int h = h0; h < h0 + 2; ++h) {
     const int smp = 16 * h + s;
     f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -455,28 +488,43 @@ __device__ __forceinline__ void grad_dx(const uint16_t* __restrict__ WT, const u
     }
   }
 }
-static_assert(kMlpHidden / 16 == kGradWaves, "grad_dx gives each wave one 16-input block");
+static_assert(kMlpHidden == 64, "grad_dx gives each wave two blocks, grad_fwd_hidden likewise");
 
-__global__ __launch_bounds__(kGradBlock) void k_mlp_grad(const uint16_t* __restrict__ wb, const uint16_t* __restrict__ wtb,
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_mlp_grad(const uint16_t* __restrict__ wb, const uint16_t* __restrict__ wtb,
                                                          const float* __restrict__ rawAll, const float* __restrict__ targetsAll,
                                                          MlpBatch batch, float* __restrict__ partials,
                                                          float* __restrict__ lossPart) {
-  __shared__ __align__(16) GradLds L;
+  __shared__ __align__(16) GradLds<WAVES> L;
+  constexpr int kTile = GradLds<WAVES>::kTile, kSmpStride = GradLds<WAVES>::kSmpStride;
+  constexpr int kGroups = kTile / 16;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int s = lane & 15, q = lane >> 4;
-  // the forward split: half h, output blocks ob0 and ob0 + 1
-  const int h = wave & 1, ob0 = 2 * (wave >> 1);
+  // the forward split: samples 16h..16h+15, output blocks ob0 and ob0 + 1
+  const int h = wave % kGroups, ob0 = 2 * (wave / kGroups);
   uint32_t first, n;
   MlpBatchRange(batch, &first, &n);
   const float* raw = rawAll + (size_t)first * kMlpRaw;
   const float* targets = targetsAll + (size_t)first * 4;
   const float invCount = n ? (float)(1.0 / (3.0 * (double)n)) : 0.0f;
-  const uint32_t tiles = (n + 31) / 32;
+  const uint32_t tiles = (n + kTile - 1) / kTile;
+  if (blockIdx.x >= tiles) return;
+  f32x4 dw0[grad_dw_blocks(WAVES, kMlpHidden, kMlpIn)], dw1[grad_dw_blocks(WAVES, kMlpHidden, kMlpHidden)],
+      dw2[grad_dw_blocks(WAVES, kMlpHidden, kMlpHidden)], dw3[grad_dw_blocks(WAVES, kMlpHidden, kMlpHidden)],
+      dw4[grad_dw_blocks(WAVES, kMlpOut, kMlpHidden)];
+  grad_zero(dw0);
+  grad_zero(dw1);
+  grad_zero(dw2);
+  grad_zero(dw3);
+  grad_zero(dw4);
+  float lossSum = 0.0f;
+  float* part = partials + (size_t)blockIdx.x * kMlpParams;
   for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    // encode: waves 0 and 1, one half each
-    if (wave < 2) {
+    const bool last = tile + gridDim.x >= tiles;  // no overflow: both are below 2^27
+    // encode: the first half of the waves, 16 samples each
+    if (wave < kGroups) {
       const int smp = 16 * h + s;
-      const uint32_t idx = tile * 32 + smp;
+      const uint32_t idx = tile * kTile + smp;
       float f[kMlpRaw];
 #pragma unroll
       for (int i = 0; i < kMlpRaw; ++i) f[i] = 0.0f;
@@ -498,17 +546,17 @@ __global__ __launch_bounds__(kGradBlock) void k_mlp_grad(const uint16_t* __restr
     }
     __syncthreads();
     // forward, keeping every layer's activations
-    grad_fwd_hidden<kMlpIn>(wb + kMlpWOff[0], L.a0, kActStride, L.a[0], L.t[0], h, ob0, lane);
+    grad_fwd_hidden<WAVES, kMlpIn>(wb + kMlpWOff[0], L.a0, kActStride, L.a[0], L.t[0], h, ob0, lane);
     __syncthreads();
 #pragma unroll 1
     for (int l = 1; l < 4; ++l) {
-      grad_fwd_hidden<kMlpHidden>(wb + kMlpWOff[l], L.a[l - 1], kHidStride, L.a[l], L.t[l], h, ob0, lane);
+      grad_fwd_hidden<WAVES, kMlpHidden>(wb + kMlpWOff[l], L.a[l - 1], kHidStride, L.a[l], L.t[l], h, ob0, lane);
       __syncthreads();
     }
-    // output layer and the loss gradient dY4 (outputs 0..2; the rest stay 0): waves 0 and 1
-    if (wave < 2) {
+    // output layer and the loss gradient dY4 (outputs 0..2; the rest stay 0): likewise
+    if (wave < kGroups) {
       const int smp = 16 * h + s;
-      const uint32_t idx = tile * 32 + smp;
+      const uint32_t idx = tile * kTile + smp;
       float loss = 0.0f;
       f32x4 y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -535,23 +583,38 @@ __global__ __launch_bounds__(kGradBlock) void k_mlp_grad(const uint16_t* __restr
       if (lane == 0) L.loss[h] = loss;
     }
     __syncthreads();
-    float* part = partials + (size_t)tile * kMlpParams;
     // layer 4: dW (16 x 64) and dX through WT_4 (64 x 32)
-    grad_dw<kMlpOut, kMlpHidden>(L.dyt[0], L.t[3], part + kMlpWOff[4], wave, lane);
-    grad_dx<32>(wtb + kMlpWTOff[4], L.dys[0], L.a[3], L.dys[1], L.dyt[1], wave, lane);
+    grad_dw<WAVES, kMlpOut, kMlpHidden>(L.dyt[0], L.t[3], dw4, last, part + kMlpWOff[4], wave, lane);
+    grad_dx<WAVES, 32>(wtb + kMlpWTOff[4], L.dys[0], L.a[3], L.dys[1], L.dyt[1], wave, lane);
     __syncthreads();
-    int cur = 1;
+    if (WAVES == 4) {  // one tile per block: nothing to keep, and less code to fetch
+      int cur = 1;
 #pragma unroll 1
-    for (int l = 3; l >= 1; --l) {
-      grad_dw<kMlpHidden, kMlpHidden>(L.dyt[cur], L.t[l - 1], part + kMlpWOff[l], wave, lane);
-      grad_dx<kMlpHidden>(wtb + kMlpWTOff[l], L.dys[cur], L.a[l - 1], L.dys[cur ^ 1], L.dyt[cur ^ 1], wave, lane);
+      for (int l = 3; l >= 1; --l) {
+        grad_zero(dw1);
+        grad_dw<WAVES, kMlpHidden, kMlpHidden>(L.dyt[cur], L.t[l - 1], dw1, true, part + kMlpWOff[l], wave, lane);
+        grad_dx<WAVES, kMlpHidden>(wtb + kMlpWTOff[l], L.dys[cur], L.a[l - 1], L.dys[cur ^ 1], L.dyt[cur ^ 1], wave,
+                                   lane);
+        __syncthreads();
+        cur ^= 1;
+      }
+    } else {
+      grad_dw<WAVES, kMlpHidden, kMlpHidden>(L.dyt[1], L.t[2], dw3, last, part + kMlpWOff[3], wave, lane);
+      grad_dx<WAVES, kMlpHidden>(wtb + kMlpWTOff[3], L.dys[1], L.a[2], L.dys[0], L.dyt[0], wave, lane);
       __syncthreads();
-      cur ^= 1;
+      grad_dw<WAVES, kMlpHidden, kMlpHidden>(L.dyt[0], L.t[1], dw2, last, part + kMlpWOff[2], wave, lane);
+      grad_dx<WAVES, kMlpHidden>(wtb + kMlpWTOff[2], L.dys[0], L.a[1], L.dys[1], L.dyt[1], wave, lane);
+      __syncthreads();
+      grad_dw<WAVES, kMlpHidden, kMlpHidden>(L.dyt[1], L.t[0], dw1, last, part + kMlpWOff[1], wave, lane);
+      grad_dx<WAVES, kMlpHidden>(wtb + kMlpWTOff[1], L.dys[1], L.a[0], L.dys[0], L.dyt[0], wave, lane);
+      __syncthreads();
     }
-    grad_dw<kMlpHidden, kMlpIn>(L.dyt[cur], L.t0, part + kMlpWOff[0], wave, lane);
-    if (threadIdx.x == 0) lossPart[tile] = L.loss[0] + L.loss[1];
+    grad_dw<WAVES, kMlpHidden, kMlpIn>(L.dyt[0], L.t0, dw0, last, part + kMlpWOff[0], wave, lane);
+    if (threadIdx.x == 0)
+      lossSum += kGroups == 4 ? (L.loss[0] + L.loss[1]) + (L.loss[2] + L.loss[3]) : L.loss[0] + L.loss[1];
     __syncthreads();
   }
+  if (threadIdx.x == 0) lossPart[blockIdx.x] = lossSum;
 }
 
 // Index into WT of parameter p = W_l[o][i].
@@ -585,30 +648,30 @@ __device__ __forceinline__ void adam_update(const MlpDev& d, int p, float g, con
   d.wbi[wi_index(p)] = b;
 }
 
-// Sum of the per-tile partials: block = 16 waves x 64 parameters; wave c
-// sums tiles c, c + 16, c + 32, ... in tile order (the loads of an unrolled
+// Sum of the partials: block = 16 waves x 64 parameters; wave c sums partials
+// c, c + 16, c + 32, ... in order (the loads of an unrolled
 // run are independent of the sum, so eight are in flight per lane), then
 // wave 0 adds the sixteen class sums as a fixed pairwise tree.  The order
-// depends only on the tile count, so a step is deterministic.  With ADAM the
+// depends only on the sample count, so a step is deterministic.  With ADAM the
 // same lane then applies the Adam step to its weight (skipped for an empty
-// batch).  Block 0 also sums the tile losses (lane l: tiles l, l + 64, ...,
+// batch).  Block 0 also sums the losses (lane l: partials l, l + 64, ...,
 // then a fixed butterfly).
 constexpr int kReduceParams = 64;
 constexpr int kReduceWaves = 16;
 template <bool ADAM>
-__global__ __launch_bounds__(64 * kReduceWaves) void k_mlp_reduce(MlpDev d, MlpBatch batch, float* __restrict__ lossOut,
-                                                                  AdamArgs adam) {
+__global__ __launch_bounds__(64 * kReduceWaves) void k_mlp_reduce(MlpDev d, MlpBatch batch, uint32_t tileLog2,
+                                                                  float* __restrict__ lossOut, AdamArgs adam) {
   __shared__ float cls[kReduceWaves][kReduceParams];
   uint32_t first, n;
   MlpBatchRange(batch, &first, &n);
-  const uint32_t tiles = (n + 31) / 32;
+  const uint32_t parts = MlpParts(n, tileLog2);
   const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;
   const uint32_t p = blockIdx.x * kReduceParams + lane;
   const float* __restrict__ partials = d.partials;
   float g = 0.0f;
   if (p < (uint32_t)kMlpParams) {
 #pragma unroll 8
-    for (uint32_t t = (uint32_t)c; t < tiles; t += kReduceWaves) g += partials[(size_t)t * kMlpParams + p];
+    for (uint32_t t = (uint32_t)c; t < parts; t += kReduceWaves) g += partials[(size_t)t * kMlpParams + p];
   }
   cls[c][lane] = g;
   __syncthreads();
@@ -625,7 +688,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void k_mlp_reduce(MlpDev d, MlpB
   }
   if (blockIdx.x == 0 && c == 0 && lossOut) {
     float l = 0.0f;
-    for (uint32_t t = (uint32_t)lane; t < tiles; t += 64) l += d.loss[t];
+    for (uint32_t t = (uint32_t)lane; t < parts; t += 64) l += d.loss[t];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
     if (lane == 0) *lossOut = l;
@@ -687,25 +750,27 @@ hipError_t LaunchMlpGradientTiles(const MlpDev& m, const float* raw, const float
   if (batch.n == 0 || batch.n > 0xffffff00u || batch.steps == 0 || batch.step >= batch.steps)
     return hipErrorInvalidValue;
   if (!batch.count && (batch.step != 0 || batch.steps != 1)) return hipErrorInvalidValue;
-  // the most tiles the batch can hold (its count is read on the device)
-  const uint32_t tiles = MlpTiles(batch.n / batch.steps);
-  if (tiles == 0 || tiles > m.partialTiles) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_mlp_grad, dim3(GridFor(tiles, 1, 4096)), dim3(kGradBlock), 0, stream, m.wb, m.wtb, raw,
-                     targets, batch, m.partials, m.loss);
+  // the most partials the batch can have (its count is read on the device)
+  const uint32_t most = batch.n / batch.steps, tileLog2 = MlpGradTileLog2(most), parts = MlpParts(most, tileLog2);
+  if (parts == 0 || parts > m.partialBlocks) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(tileLog2 == 6 ? k_mlp_grad<8> : k_mlp_grad<4>, dim3(parts), dim3(8u << tileLog2), 0, stream, m.wb,
+                     m.wtb, raw, targets, batch, m.partials, m.loss);
   return hipGetLastError();
 }
 
 hipError_t LaunchMlpReduce(const MlpDev& m, const MlpBatch& batch, float* lossOut, const AdamParams* adam,
                            hipStream_t stream) {
   const dim3 grid((kMlpParams + kReduceParams - 1) / kReduceParams), block(64 * kReduceWaves);
+  if (batch.steps == 0) return hipErrorInvalidValue;
+  const uint32_t tileLog2 = MlpGradTileLog2(batch.n / batch.steps);
   if (!adam) {
-    hipLaunchKernelGGL(k_mlp_reduce<false>, grid, block, 0, stream, m, batch, lossOut, AdamArgs{});
+    hipLaunchKernelGGL(k_mlp_reduce<false>, grid, block, 0, stream, m, batch, tileLog2, lossOut, AdamArgs{});
     return hipGetLastError();
   }
   const double bc1 = 1.0 - std::pow((double)adam->beta1, (double)adam->step);
   const double bc2 = 1.0 - std::pow((double)adam->beta2, (double)adam->step);
   const AdamArgs a{adam->lr, adam->beta1, adam->beta2, adam->eps, (float)bc1, (float)bc2};
-  hipLaunchKernelGGL(k_mlp_reduce<true>, grid, block, 0, stream, m, batch, lossOut, a);
+  hipLaunchKernelGGL(k_mlp_reduce<true>, grid, block, 0, stream, m, batch, tileLog2, lossOut, a);
   return hipGetLastError();
 }
 

@@ -83,6 +83,26 @@ def test_gradient_matches_oracle(mctx, n):
     assert (g[mlp.W_OFF[4] + 3 * 64:] == 0).all()
 
 
+@pytest.mark.parametrize("n", [33, 2048, 2049, 16384, 16385, 40001])
+def test_gradient_at_tile_and_block_edges(mctx, n):
+    """Tiles of 32 samples up to 2,048, of 64 above, at most 256 blocks: a tile
+    with a remainder, both sides of the rule, one tile per block, and blocks with
+    two and three tiles.  The loss is a sum of
+    squares and the layers' weights and activations have 8 significant bits, so
+    the bounds are those of test_gradient_matches_oracle."""
+    f = features(n, 7 + n)
+    t = smooth_target(f)
+    w = mctx.mlp_get_weights()
+    g, loss = mctx.mlp_gradient(f, t)
+    lref, gref = mlp.loss_and_gradient(w, mlp.encode(f), t)
+    assert loss == pytest.approx(lref, rel=1e-2)
+    for l in range(5):
+        a, b = g[mlp.W_OFF[l]:mlp.W_OFF[l + 1]], gref[mlp.W_OFF[l]:mlp.W_OFF[l + 1]]
+        assert np.linalg.norm(a - b) < 3e-2 * np.linalg.norm(b), l
+    g2, loss2 = mctx.mlp_gradient(f, t)
+    assert np.array_equal(g.view(np.uint32), g2.view(np.uint32)) and loss == loss2
+
+
 def test_gradient_is_deterministic(mctx):
     f = features(3000, 5)
     t = smooth_target(f)
