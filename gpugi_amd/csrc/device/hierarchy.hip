@@ -172,9 +172,10 @@ __device__ void count_hits(const RefScene& s, gg::V3 o, gg::V3 d, float rayLengt
   } while (node != 0 || nextIsLeaf);
 }
 
-// Eight waves per SIMD (64 VGPRs, a 48-byte spill) instead of five (88 VGPRs,
-// no spill): the two walks per ray wait on memory, and the extra waves cover
-// it (93 against 123 ms per 10-pass update on a 2M-triangle heightfield).
+// Eight waves per SIMD (64 VGPRs, with a spill) instead of five (without one):
+// the two walks per ray wait on memory, and the extra waves cover it (39.7 ms per
+// 10-pass update of a 524,288-triangle heightfield at 1280x720; 41.8, 43.6 and 47.9
+// with seven, six and five waves).
 __global__ __launch_bounds__(kHierBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_hier_acquire(
     DrawParams p, uint32_t frameSeed, unsigned long long* __restrict__ imp, uint32_t numNodes, uint32_t tilesW,
     uint32_t numPixels) {
