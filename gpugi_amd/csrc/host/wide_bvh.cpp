@@ -284,8 +284,10 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
   }
   // Worst-case stack.  A visit goes on with one hit inner child; the other hit
   // inner children wait in one entry, and the hit leaves in another when both
-  // pending-leaf slots of the lane are taken, so
-  //   stack(n) = [n has two inner children] + [n has a leaf] + max stack(inner child).
+  // pending-leaf slots of the lane are taken.  An unused slot counts as a leaf: from
+  // about 10^6 of the node's extents away the slack of the slab test lets its
+  // inverted box through.  So
+  //   stack(n) = [n has two inner children] + [a slot of n is no inner child] + max stack(inner child).
   // An entry that waits keeps its place while children of it are visited, which
   // the sum covers.  Children are numbered after their parents.
   std::vector<uint32_t> stack(out->nodes.size(), 0), pending(out->nodes.size(), 0), depth(out->nodes.size(), 1);
@@ -302,7 +304,7 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
       pending[i] = std::max(pending[i], pending[c]);
       depth[i] = std::max(depth[i], depth[c] + 1);
     }
-    stack[i] += (numInner > 1 ? 1 : 0) + (leaves > 0 ? 1 : 0);
+    stack[i] += (numInner > 1 ? 1 : 0) + (numInner < (uint32_t)W ? 1 : 0);
     pending[i] += numInner + leaves - (numInner > 0 ? 1 : 0);
   }
   out->maxStack = stack[0];

@@ -85,6 +85,71 @@ def centre_rays(n, seed):
     return rays
 
 
+class TreeScene:
+    """A scene with a hierarchy of its own: tree is a nested tuple (lo, hi, list of children, or array of a leaf's
+    one or two triangles), boxes at least as large as what they hold."""
+
+    def __init__(self, tree):
+        nodes, tris, pos = [], [], []
+
+        def put(node, escape):
+            lo, hi, kids = node
+            i = len(nodes)
+            nodes.append([lo, i + 1, hi, escape])
+            if isinstance(kids, np.ndarray):
+                nodes[i][1] = 0x80000000 | (len(tris) // 2)
+                for t in kids:
+                    tris.append([len(pos), len(pos) + 1, len(pos) + 2, 0])
+                    pos.extend(t)
+                tris.extend([[0, 0, 0, 0]] * (2 - len(kids)))
+                return
+            for k, kid in enumerate(kids):
+                put(kid, escape if k + 1 == len(kids) else len(nodes) + size(kid))
+
+        def size(node):
+            return 1 if isinstance(node[2], np.ndarray) else 1 + sum(size(k) for k in node[2])
+
+        put(tree, 0)
+        h = np.zeros((len(nodes), 8), np.float32)
+        h[:, 0:3], h[:, 4:7] = [n[0] for n in nodes], [n[2] for n in nodes]
+        h.view(np.uint32)[:, 3], h.view(np.uint32)[:, 7] = [n[1] for n in nodes], [n[3] for n in nodes]
+        self.a = {"hierarchy": h, "triangles": np.array(tris, np.int32), "positions": np.array(pos, np.float32),
+                  "vertex_info": np.zeros((len(pos), 4), np.float32), "materials": np.zeros(1, _rt.MATERIAL_DTYPE),
+                  "triangles_per_leaf": 2}
+
+    def arrays(self):
+        return self.a
+
+    def desc(self):
+        a = self.a
+        return _rt.SceneDesc(a["hierarchy"].ctypes.data, len(a["hierarchy"]), a["triangles"].ctypes.data,
+                             len(a["triangles"]) // 2, 2, a["positions"].ctypes.data, a["vertex_info"].ctypes.data,
+                             len(a["positions"]), a["materials"].ctypes.data, len(a["materials"]))
+
+
+def five_ary_chain(levels, seed):
+    """Wide nodes with five inner children, three unused slots and no leaf: per level four nodes of five leaves
+    (opening one would take a ninth slot) and the next level, whose box is the largest.  All of it within half a
+    unit of the origin; small triangles near its middle that face (1, 1, 1)."""
+    rng = np.random.default_rng(seed)
+    plane = np.linalg.qr(np.array([[1.0, 1.0, 1.0], [1.0, 0.0, 0.0], [0.0, 1.0, 0.0]]).T)[0][:, 1:].T
+
+    def box(r):
+        return (np.full(3, -r), np.full(3, r))
+
+    def leaf():
+        c = 0.2 * (rng.random(3) - 0.5)
+        return (*box(0.25), c + 0.2 * (rng.random((2, 3, 2)) - 0.5) @ plane)
+
+    def fan():
+        return (*box(0.3), [leaf() for _ in range(5)])
+
+    node = fan()
+    for _ in range(levels):
+        node = (*box(0.5), [fan() for _ in range(4)] + [node])
+    return TreeScene(node)
+
+
 SCENES = {"cornell": _rt.HostScene.cornell, "heightfield": lambda: _rt.HostScene.heightfield(20, 7),
           "clutter": lambda: _rt.HostScene.clutter(3, 5), "nested": lambda: nested_scene(30),
           "triangle": lambda: _rt.HostScene.build([[0, 0, 0], [1, 0, 0.2], [0, 1, 0.1]], [[0, 1, 2]])}
@@ -124,3 +189,28 @@ def test_deep_tree_uses_the_spill_stack(walk, oracle):
     assert n["used"] > 48
     got, n = walk(hs, rays, 1, any_hit=True, lds=10)
     assert np.array_equal(got[:, 0], oracle.bruteforce(sc, rays, any_hit=True)[:, 0])
+
+
+@pytest.mark.parametrize("distance", [3e5, 3e6, 1e7])
+def test_far_rays_stay_within_the_stack_bound(walk, oracle, distance):
+    """From about 1e6 of a node's extents away, the slack that covers the rounding of the slab distances is
+    larger than the node, and the inverted boxes of its unused slots pass like any other.  Both queries then have
+    an empty leaf group at every node of the chain, on top of the children that wait; the walk must have the
+    entries for them, with the shipped ten in LDS as with one."""
+    hs = five_ary_chain(14, 2)
+    sc = oracle.Scene(hs.arrays())
+    rng = np.random.default_rng(4)
+    n = 300
+    rays = np.zeros((n, 8), np.float32)
+    d = (1.0 + 0.2 * rng.random((n, 3))) * rng.choice([-1.0, 1.0], (n, 1))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays[:, 0:3], rays[:, 3], rays[:, 4:7] = 3.0 * rng.random((n, 3)) - 1.5 - distance * d, 3.0 * distance, d
+    want = oracle.bruteforce(sc, rays)
+    want_any = oracle.bruteforce(sc, rays, any_hit=True)[:, 0]
+    assert 0 < want_any.sum() < n
+    for leaf in (1, 2):
+        for lds in (10, 1):
+            got, _ = walk(hs, rays, leaf, lds=lds)
+            assert np.array_equal(got, want), (leaf, lds)
+            got, _ = walk(hs, rays, leaf, any_hit=True, lds=lds)
+            assert np.array_equal(got[:, 0], want_any), (leaf, lds)
