@@ -138,7 +138,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)
     source.sceneBase = sl.tileBase;
     source.sceneEnd = sl.tileBase + sl.tilesX * sl.tilesY;
     prog.params = &sl.p;
-    phased_paths<false, S>(sl.p.wide, stk, spill, sl.tilesX * sl.tilesY * kTileThreads, source, (uint32_t)kTileThreads,
+    const WideScene ws = sl.p.wide;
+    phased_paths<false, S>(ws, stk, spill, sl.tilesX * sl.tilesY * kTileThreads, source, (uint32_t)kTileThreads,
                            prog);
   }
   // one atomic per wave
@@ -428,6 +429,7 @@ int gpugi_batch_finalize(gpugi_batch* b) {
     p.wide.spillDepth = b->spillDepth;
     p.wide.numThreads = 0;
     p.wide.errorFlag = &b->dCounters->pad;
+    SetWideScale(&p.wide, s.wide.tScale);
     p.camera = s.camera;
     p.width = s.width;
     p.height = s.height;

@@ -53,6 +53,7 @@ struct gpugi_ctx {
   void* dWideQueue = nullptr;  // the wide trace kernel's batch counters
   size_t spillBytes = 0;
   uint32_t wideMaxStack = 0, wideMaxPending = 0, wideNumNodes = 0;
+  float wideTScale = 1.0f;
   std::map<int, int> wideBlocksPerCU;  // per LDS stack depth: resident blocks of the trace kernel
   int wideLeaf = 2;     // triangles per merged wide leaf
   int wideStack = 10;   // LDS stack entries per lane of the trace kernel
@@ -190,6 +191,7 @@ WideScene MakeWide(const gpugi_ctx* c, int stack) {
   s.numThreads = 0;
   s.errorFlag = (uint32_t*)c->dCounters + 1;
   s.queue = (uint32_t*)c->dWideQueue;
+  SetWideScale(&s, c->wideTScale);
   return s;
 }
 
@@ -275,6 +277,7 @@ int RebuildWide(gpugi_ctx* ctx) {
                            hipMemcpyHostToDevice));
   ctx->wideMaxStack = wide.maxStack;
   ctx->wideMaxPending = wide.maxPending;
+  ctx->wideTScale = wide.tScale;
   ctx->wideNumNodes = (uint32_t)wide.nodes.size();
   ctx->hasWide = true;
   return GPUGI_OK;

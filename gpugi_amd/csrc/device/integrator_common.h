@@ -203,7 +203,7 @@ __device__ __forceinline__ void phased_paths(const WideScene& ws, uint2* lds, ui
         mode = kIdle;
       } else {
         const bool any = next == kPathOccludes;
-        wide_init<WT>(st, any ? prog.lo : prog.o, any ? prog.ld : prog.d, any ? prog.ltmax : gg::kRayMax);
+        wide_init<WT>(ws, st, any ? prog.lo : prog.o, any ? prog.ld : prog.d, any ? prog.ltmax : gg::kRayMax);
         st.anyHit = any;
         mode = kTraces;
       }

@@ -86,7 +86,7 @@ struct WideStack {
 
 struct WideState {
   gg::V3 o, d;
-  float ix, iy, iz;
+  float ix, iy, iz;  // 1/d times WideScene::tScale, so slab and entry distances are scaled, tbest is not
   float tbest;
   int bestSlot;
   float bu, bv;
@@ -103,8 +103,7 @@ struct WideState {
 // below 2^-23 scales every slab distance of a ray by the same factor (1 + δ),
 // which the far-distance and hit-distance widening of 1 + 2^-20 covers.
 __device__ __forceinline__ float safe_inv(float d) {
-  const float tiny = 1e-20f;
-  return __builtin_amdgcn_rcpf(fabsf(d) > tiny ? d : copysignf(tiny, d));
+  return __builtin_amdgcn_rcpf(copysignf(fmaxf(fabsf(d), 1e-20f), d));  // (NaN: 1e-20)
 }
 
 // Two quantized planes as 16-bit integers: bytes i and i + 1 of `lo` or of `hi`,
@@ -128,12 +127,12 @@ __device__ __forceinline__ float plane_fma(uint32_t pair, int half, float A24, f
 }
 
 template <bool WT = false>
-__device__ __forceinline__ void wide_init(WideState& st, gg::V3 o, gg::V3 d, float tmax) {
+__device__ __forceinline__ void wide_init(const WideScene& s, WideState& st, gg::V3 o, gg::V3 d, float tmax) {
   st.o = o;
   st.d = d;
-  st.ix = safe_inv(d.x);
-  st.iy = safe_inv(d.y);
-  st.iz = safe_inv(d.z);
+  st.ix = safe_inv(d.x) * s.tScale;
+  st.iy = safe_inv(d.y) * s.tScale;
+  st.iz = safe_inv(d.z) * s.tScale;
   st.tbest = tmax;
   st.bestSlot = -1;
   st.bu = st.bv = 0.0f;
@@ -203,7 +202,8 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
   // B_a + |B_a| * 2^-20 + |A_a| * 2^-12: along every ray into a box, t is at most
   // |B_a| + 255 |A_a| for each far plane, so this covers the axes' different δ_a
   // (2^-22 t), the roundings of B_a (2^-23 |B_a|) and those of both fmas (2^-24 t
-  // each).  The bytes giving the near planes (lo or hi) are picked per axis by the
+  // each).  (inv_a, so every distance here, is times s.tScale, a power of two that is 1
+  // but for scenes whose A_a * 2^24 could overflow.)  The bytes giving the near planes (lo or hi) are picked per axis by the
   // sign of inv_a.  The host checks in extended precision that origin + q * s
   // encloses every child box, so with the hit distance widened by 1 + 2^-20 a box
   // that holds the closest hit is never rejected (the argument of Ize 2013,
@@ -218,7 +218,7 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
               bfz = __builtin_fmaf(fabsf(Az), kQuantumSlack, __builtin_fmaf(fabsf(Bz), kFarSlack, Bz));
   constexpr float k2p24 = 16777216.0f;
   const float Ax24 = Ax * k2p24, Ay24 = Ay * k2p24, Az24 = Az * k2p24;
-  const float tbScaled = st.tbest * 1.00000095f;
+  const float tbScaled = st.tbest * s.hitScale;
   const uint32_t selX = st.ix < 0.0f ? kPlaneHi : kPlaneLo, selY = st.iy < 0.0f ? kPlaneHi : kPlaneLo,
                  selZ = st.iz < 0.0f ? kPlaneHi : kPlaneLo;
   // A hit child's key is its entry distance with the three lowest bits replaced
@@ -352,8 +352,8 @@ __device__ __forceinline__ void wide_leaf(const WideScene& s, WideState& st) {
 // hit until one yields a node, or a leaf group finds both pending slots taken
 // (the entry stays), or the stack is empty.
 template <int Q, int B, int S>
-__device__ __forceinline__ void wide_pop(WideState& st, const WideStack& stk) {
-  const float tb = st.tbest * 1.00000095f;  // entry distances are lower bounds with this slack
+__device__ __forceinline__ void wide_pop(const WideScene& s, WideState& st, const WideStack& stk) {
+  const float tb = st.tbest * s.hitScale;  // entry distances are lower bounds with this slack
   int sp = st.sp;
   uint32_t node = kWideNoNode;
   while (sp > 0) {
@@ -403,7 +403,7 @@ __device__ __forceinline__ bool wide_pass(const WideScene& s, WideState& st, boo
     if (!wide_visit<Q, B, S>(s, st, stk)) return true;  // overflow, slot -2
   }
   if (st.node == kWideNoNode) {
-    wide_pop<Q, B, S>(st, stk);
+    wide_pop<Q, B, S>(s, st, stk);
     return st.node == kWideNoNode && st.leafMask == 0u;
   }
   return false;
@@ -417,7 +417,7 @@ __device__ __forceinline__ WideResult trace_wide_ray(const WideScene& s, gg::V3 
                                                      uint2* lds, int tid, uint2* spill) {
   const WideStack stk{as_lds(lds), tid, spill, 1u};
   WideState st;
-  wide_init<WT>(st, o, d, tmax);
+  wide_init<WT>(s, st, o, d, tmax);
   bool live = true;
   for (;;) {
     const uint64_t act = __ballot(live);

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(7))) void k_t
         else if (next < bEnd) r = (uint64_t)next * 64u + (rank - avail);
         if (r < n) {
           const float4 r0 = rays[2 * (size_t)r], r1 = rays[2 * (size_t)r + 1];
-          wide_init<WT>(st, gg::v3(r0.x, r0.y, r0.z), gg::v3(r1.x, r1.y, r1.z), r0.w);
+          wide_init<WT>(s, st, gg::v3(r0.x, r0.y, r0.z), gg::v3(r1.x, r1.y, r1.z), r0.w);
           ri = (uint32_t)r;
           active = true;
         }

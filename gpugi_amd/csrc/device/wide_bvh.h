@@ -65,7 +65,11 @@ struct WideBVHHost {
   uint32_t maxPending = 0;  // most children that can wait on a traversal stack (siblings summed along a path)
   uint32_t maxStack = 0;    // most stack entries those take (an entry holds the waiting children of one node)
   uint32_t depth = 0;
+  // Slab distances are computed times this power of two: 1, or less where a node's quantum exceeds 2^36
+  // (wide_visit multiplies by up to 2^24 / 1e-20 * quantum, which has to stay finite).
+  float tScale = 1.0f;
 };
+constexpr int kWideQuantumLog2 = 36;
 
 // Re-packs the reference BVH2 (any arity up to 8 written in preorder with escape
 // pointers) into the 8-wide quantized layout.  Leaves of up to
@@ -88,7 +92,13 @@ struct WideScene {
   uint32_t numThreads;                // persistent threads the spill buffer is sized for
   uint32_t* errorFlag;                // set to nonzero if a stack would overflow
   uint32_t* queue;                    // kWideQueueWords: the trace kernel's per-XCD batch counters
+  float tScale;                       // WideBVHHost::tScale
+  float hitScale;                     // tScale * (1 + 2^-20): scales and widens the hit distance
 };
+inline void SetWideScale(WideScene* s, float tScale) {
+  s->tScale = tScale;
+  s->hitScale = tScale * 1.00000095f;
+}
 constexpr int kWideQueueStride = 32;  // counters 128 bytes apart
 constexpr int kWideQueueWords = 8 * kWideQueueStride;
 #endif

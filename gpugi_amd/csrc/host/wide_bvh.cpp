@@ -211,6 +211,7 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
     uint32_t wideIndex;  // index of the wide node to fill
   };
   std::vector<Pending> todo;
+  uint32_t largest = 0;  // biased exponent of the largest quantum
   out->nodes.push_back(WideNodeHost());
   todo.push_back({0, 0});
   while (!todo.empty()) {
@@ -266,6 +267,7 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
         if (ok) break;
       }
       biased[a] = (uint32_t)b;
+      largest = std::max(largest, biased[a]);
     }
     uint32_t inner = 0, numInner = 0;
     for (size_t s = 0; s < (size_t)W; ++s) {
@@ -282,6 +284,7 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
     node.exps = biased[0] | (biased[1] << 8) | (biased[2] << 16) | (inner << 24);
     out->nodes[p.wideIndex] = node;
   }
+  out->tScale = std::ldexp(1.0f, std::min(0, 127 + kWideQuantumLog2 - (int)largest));
   // Worst-case stack.  A visit goes on with one hit inner child; the other hit
   // inner children wait in one entry, and the hit leaves in another when both
   // pending-leaf slots of the lane are taken.  An unused slot counts as a leaf: from

@@ -86,6 +86,7 @@ extern "C" int wide_walk(const gpugi_scene_desc* d, uint32_t leaf, int any, int 
   s.tris = (const float4*)b.tris.data();
   s.spillDepth = b.maxStack > (uint32_t)ldsEntries ? b.maxStack - (uint32_t)ldsEntries : 0;
   s.errorFlag = &flag;
+  SetWideScale(&s, b.tScale);
   std::vector<uint2> lds((size_t)ldsEntries * kLanes, uint2{0xdeadu, 0xdeadu});
   std::vector<uint2> spill(s.spillDepth, uint2{0xdeadu, 0xdeadu});
   if (ldsEntries == 1) TraceS<1>(any != 0, wt != 0, s, rays, hits, n, &lds, &spill);

@@ -85,7 +85,27 @@ def centre_rays(n, seed):
     return rays
 
 
-class TreeScene:
+class ArrayScene:
+    """A scene given by its reference-layout arrays."""
+
+    def __init__(self, arrays):
+        self.a = arrays
+
+    def arrays(self):
+        return self.a
+
+    def info(self):
+        root = self.a["hierarchy"][0]
+        return {"bbox_min": root[0:3].astype(np.float64), "bbox_max": root[4:7].astype(np.float64)}
+
+    def desc(self):
+        a = self.a
+        return _rt.SceneDesc(a["hierarchy"].ctypes.data, len(a["hierarchy"]), a["triangles"].ctypes.data,
+                             len(a["triangles"]) // 2, 2, a["positions"].ctypes.data, a["vertex_info"].ctypes.data,
+                             len(a["positions"]), a["materials"].ctypes.data, len(a["materials"]))
+
+
+class TreeScene(ArrayScene):
     """A scene with a hierarchy of its own: tree is a nested tuple (lo, hi, list of children, or array of a leaf's
     one or two triangles), boxes at least as large as what they hold."""
 
@@ -113,18 +133,10 @@ class TreeScene:
         h = np.zeros((len(nodes), 8), np.float32)
         h[:, 0:3], h[:, 4:7] = [n[0] for n in nodes], [n[2] for n in nodes]
         h.view(np.uint32)[:, 3], h.view(np.uint32)[:, 7] = [n[1] for n in nodes], [n[3] for n in nodes]
-        self.a = {"hierarchy": h, "triangles": np.array(tris, np.int32), "positions": np.array(pos, np.float32),
-                  "vertex_info": np.zeros((len(pos), 4), np.float32), "materials": np.zeros(1, _rt.MATERIAL_DTYPE),
-                  "triangles_per_leaf": 2}
-
-    def arrays(self):
-        return self.a
-
-    def desc(self):
-        a = self.a
-        return _rt.SceneDesc(a["hierarchy"].ctypes.data, len(a["hierarchy"]), a["triangles"].ctypes.data,
-                             len(a["triangles"]) // 2, 2, a["positions"].ctypes.data, a["vertex_info"].ctypes.data,
-                             len(a["positions"]), a["materials"].ctypes.data, len(a["materials"]))
+        super().__init__({"hierarchy": h, "triangles": np.array(tris, np.int32),
+                          "positions": np.array(pos, np.float32),
+                          "vertex_info": np.zeros((len(pos), 4), np.float32),
+                          "materials": np.zeros(1, _rt.MATERIAL_DTYPE), "triangles_per_leaf": 2})
 
 
 def five_ary_chain(levels, seed):
@@ -214,3 +226,28 @@ def test_far_rays_stay_within_the_stack_bound(walk, oracle, distance):
             assert np.array_equal(got, want), (leaf, lds)
             got, _ = walk(hs, rays, leaf, any_hit=True, lds=lds)
             assert np.array_equal(got[:, 0], want_any), (leaf, lds)
+
+
+@pytest.mark.parametrize("log2", [-10, 30, 40, 44, 47, 50, 56])
+def test_walk_in_scaled_scenes(walk, oracle, log2):
+    """The heightfield times a power of two, up to extents of 10^18, on rays of which a quarter are parallel to an
+    axis, most of those vertical: their reciprocal of 1e20 times a node's quantum must not overflow."""
+    a = _rt.HostScene.heightfield(20, 7).arrays()
+    k = np.float32(2.0 ** log2)
+    a["positions"] *= k
+    a["hierarchy"][:, [0, 1, 2, 4, 5, 6]] *= k
+    hs = ArrayScene(a)
+    sc = oracle.Scene(a)
+    rays = ray_set(hs, 2000, 13)
+    rays[:400, 4:7] = 0.0
+    rays[:400, 5] = np.where(np.arange(400) % 2, 1.0, -1.0)
+    rays[:400, 1] = rays[:400, 5] * -2.0 * k
+    rays[:400, 3] = np.float32(3.402823466e38)
+    want = oracle.bruteforce(sc, rays)
+    want_any = oracle.bruteforce(sc, rays, any_hit=True)[:, 0]
+    assert 100 < (want[:400, 0] >= 0).sum() < 400
+    for lds in (10, 1):
+        got, _ = walk(hs, rays, 2, lds=lds)
+        assert np.array_equal(got, want), np.nonzero((got != want).any(1))[0][:5]
+        got, _ = walk(hs, rays, 2, any_hit=True, lds=lds)
+        assert np.array_equal(got[:, 0], want_any)
