@@ -126,6 +126,8 @@ __device__ __forceinline__ float plane_fma(uint32_t pair, int half, float A24, f
 #endif
 }
 
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
+
 template <bool WT = false>
 __device__ __forceinline__ void wide_init(const WideScene& s, WideState& st, gg::V3 o, gg::V3 d, float tmax) {
   st.o = o;
@@ -142,6 +144,13 @@ __device__ __forceinline__ void wide_init(const WideScene& s, WideState& st, gg:
   st.sp = 0;
   st.found = false;
   if (WT) st.wr = wt_setup(d);
+  // A ray without a finite origin component, or with a NaN for its length, hits nothing,
+  // but minima and maxima drop the NaNs of its slab distances: they would let every box
+  // through.  Here the scene lies behind it, so that its walk ends at the root.
+  if (!(finite(o.x) || finite(o.y) || finite(o.z)) || tmax != tmax) {
+    st.o.x = 1e38f;
+    st.ix = s.tScale;
+  }
 }
 
 // The node in slot `slot` of the node whose inner children (mask `inner`) start at `first`.
@@ -203,11 +212,11 @@ __device__ __forceinline__ bool wide_visit(const WideScene& s, WideState& st, co
   // |B_a| + 255 |A_a| for each far plane, so this covers the axes' different δ_a
   // (2^-22 t), the roundings of B_a (2^-23 |B_a|) and those of both fmas (2^-24 t
   // each).  (inv_a, so every distance here, is times s.tScale, a power of two that is 1
-  // but for scenes whose A_a * 2^24 could overflow.)  The bytes giving the near planes (lo or hi) are picked per axis by the
-  // sign of inv_a.  The host checks in extended precision that origin + q * s
-  // encloses every child box, so with the hit distance widened by 1 + 2^-20 a box
-  // that holds the closest hit is never rejected (the argument of Ize 2013,
-  // "Robust BVH ray traversal").
+  // but for scenes whose A_a * 2^24 could overflow.)  The bytes giving the near planes
+  // (lo or hi) are picked per axis by the sign of inv_a.  The host checks in extended
+  // precision that origin + q * s encloses every child box, so with the hit distance
+  // widened by 1 + 2^-20 a box that holds the closest hit is never rejected (the
+  // argument of Ize 2013, "Robust BVH ray traversal").
   const float Ax = sx * st.ix, Ay = sy * st.iy, Az = sz * st.iz;
   const float Bx = (ox - o.x) * st.ix, By = (oy - o.y) * st.iy, Bz = (oz - o.z) * st.iz;
   constexpr float kNearSlack = 4.76837158e-7f, kFarSlack = 9.53674316e-7f, kQuantumSlack = 2.44140625e-4f;

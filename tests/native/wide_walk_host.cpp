@@ -20,7 +20,9 @@ static inline int __popcll(uint64_t x) { return __builtin_popcountll(x); }
 static inline uint64_t __ballot(bool b) { return b ? 1u : 0u; }
 static inline uint32_t atomicOr(uint32_t* p, uint32_t v) { const uint32_t o = *p; *p |= v; return o; }
 static inline float amd_rcp(float x) { return 1.0f / x; }
+static uint32_t slots_tested;  // the walk shifts in one bit per child box
 static inline uint32_t amd_alignbit(uint32_t hi, uint32_t lo, uint32_t n) {
+  ++slots_tested;
   return (uint32_t)((((uint64_t)hi << 32) | lo) >> (n & 31u));
 }
 // bytes 0-3 of a selector byte are lo's, 4-7 hi's, 0x0c is zero
@@ -74,10 +76,10 @@ void TraceS(bool any, bool wt, const WideScene& s, const float* rays, int32_t* h
 }  // namespace
 
 // Traces n rays (8 floats each) into hits (4 words each).  counts: {nodes, triangles,
-// max pending, max stack entries, entries the deepest ray used, overflow flag}.
+// max pending, max stack entries, entries the deepest ray used, overflow flag, nodes visited}.
 // ldsEntries: 1 or 10.  Returns 0, or 1 if the tree could not be built.
 extern "C" int wide_walk(const gpugi_scene_desc* d, uint32_t leaf, int any, int wt, int ldsEntries, const float* rays,
-                         int32_t* hits, size_t n, uint32_t counts[6]) {
+                         int32_t* hits, size_t n, uint32_t counts[7]) {
   WideBVHHost b;
   if (!BuildWideBVH(*d, leaf, &b, wt != 0).empty()) return 1;
   uint32_t flag = 0;
@@ -89,6 +91,7 @@ extern "C" int wide_walk(const gpugi_scene_desc* d, uint32_t leaf, int any, int 
   SetWideScale(&s, b.tScale);
   std::vector<uint2> lds((size_t)ldsEntries * kLanes, uint2{0xdeadu, 0xdeadu});
   std::vector<uint2> spill(s.spillDepth, uint2{0xdeadu, 0xdeadu});
+  slots_tested = 0;
   if (ldsEntries == 1) TraceS<1>(any != 0, wt != 0, s, rays, hits, n, &lds, &spill);
   else TraceS<10>(any != 0, wt != 0, s, rays, hits, n, &lds, &spill);
   counts[0] = (uint32_t)b.nodes.size();
@@ -99,5 +102,6 @@ extern "C" int wide_walk(const gpugi_scene_desc* d, uint32_t leaf, int any, int 
   for (int e = 0; e < ldsEntries; ++e) counts[4] += lds[(size_t)e * kLanes + 1].x != 0xdeadu;
   for (const uint2& e : spill) counts[4] += e.x != 0xdeadu;
   counts[5] = flag;
+  counts[6] = slots_tested / kWideArity;
   return 0;
 }

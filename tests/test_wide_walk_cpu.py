@@ -29,12 +29,12 @@ def walk(tmp_path_factory):
 
     def run(scene, rays, leaf=2, any_hit=False, watertight=False, lds=10):
         rays = np.ascontiguousarray(rays, np.float32)
-        hits, counts = np.zeros((len(rays), 4), np.int32), np.zeros(6, np.uint32)
+        hits, counts = np.zeros((len(rays), 4), np.int32), np.zeros(7, np.uint32)
         p = ctypes.c_void_p
         assert fn(ctypes.byref(scene.desc()), ctypes.c_uint32(leaf), int(any_hit), int(watertight), lds,
                   p(rays.ctypes.data), p(hits.ctypes.data), ctypes.c_size_t(len(rays)), p(counts.ctypes.data)) == 0
         assert counts[5] == 0 and counts[4] <= counts[3]  # no overflow, the stack bound holds
-        return hits, dict(zip(("nodes", "tris", "pending", "stack", "used"), counts.tolist()))
+        return hits, dict(zip(("nodes", "tris", "pending", "stack", "used", "flag", "visits"), counts.tolist()))
     return run
 
 
@@ -251,3 +251,19 @@ def test_walk_in_scaled_scenes(walk, oracle, log2):
         assert np.array_equal(got, want), np.nonzero((got != want).any(1))[0][:5]
         got, _ = walk(hs, rays, 2, any_hit=True, lds=lds)
         assert np.array_equal(got[:, 0], want_any)
+
+
+@pytest.mark.parametrize("watertight", [False, True])
+def test_rays_that_cannot_hit_end_at_the_root(walk, watertight):
+    """Origins of NaN and infinities only, and NaN ray lengths: a miss with the ray's own length, after the
+    root's boxes (of which the walk's first visit tests all)."""
+    hs = _rt.HostScene.heightfield(20, 7)
+    rays = ray_set(hs, 400, 17)
+    rng = np.random.default_rng(5)
+    rays[:300, 0:3] = rng.choice(np.array([np.nan, -np.nan, np.inf, -np.inf], np.float32), (300, 3))
+    rays[300:, 3] = np.nan
+    for any_hit in (False, True):
+        got, n = walk(hs, rays, 2, any_hit=any_hit, watertight=watertight)
+        assert (got[:, 0] == (0 if any_hit else -1)).all()
+        assert any_hit or np.array_equal(got[:, 1], rays[:, 3].view(np.int32))
+        assert n["visits"] == len(rays)
