@@ -52,7 +52,7 @@ struct gpugi_ctx {
   void* dCounters = nullptr;  // [0] ray counter, [1] error flag, [2] hit count
   void* dWideQueue = nullptr;  // the wide trace kernel's batch counters
   size_t spillBytes = 0;
-  uint32_t wideMaxStack = 0, wideMaxPending = 0, wideNumNodes = 0;
+  uint32_t wideMaxStack = 0, wideNumNodes = 0;
   float wideTScale = 1.0f;
   std::map<int, int> wideBlocksPerCU;  // per LDS stack depth: resident blocks of the trace kernel
   int wideLeaf = 2;     // triangles per merged wide leaf
@@ -276,7 +276,6 @@ int RebuildWide(gpugi_ctx* ctx) {
     HIP_TRY(ctx, hipMemcpy(ctx->dWideTris, wide.tris.data(), wide.tris.size() * sizeof(WideTriHost),
                            hipMemcpyHostToDevice));
   ctx->wideMaxStack = wide.maxStack;
-  ctx->wideMaxPending = wide.maxPending;
   ctx->wideTScale = wide.tScale;
   ctx->wideNumNodes = (uint32_t)wide.nodes.size();
   ctx->hasWide = true;
@@ -1380,7 +1379,7 @@ int gpugi_get_wide_config(gpugi_ctx* ctx, int* max_leaf_triangles, int* lds_stac
   if (lds_stack_entries) *lds_stack_entries = ctx->wideStack;
   if (refill_lanes) *refill_lanes = ctx->wideRefill;
   if (wait_lanes) *wait_lanes = ctx->wideWait;
-  if (max_stack) *max_stack = ctx->wideMaxPending;
+  if (max_stack) *max_stack = ctx->wideMaxStack;
   return GPUGI_OK;
 }
 

@@ -62,8 +62,7 @@ static_assert(sizeof(WideTriHost) == 48, "wide triangle is 48 bytes");
 struct WideBVHHost {
   std::vector<WideNodeHost> nodes;
   std::vector<WideTriHost> tris;
-  uint32_t maxPending = 0;  // most children that can wait on a traversal stack (siblings summed along a path)
-  uint32_t maxStack = 0;    // most stack entries those take (an entry holds the waiting children of one node)
+  uint32_t maxStack = 0;  // most traversal stack entries of a ray (one holds the waiting children of a node)
   uint32_t depth = 0;
   // Slab distances are computed times this power of two: 1, or less where a node's quantum exceeds 2^36
   // (wide_visit multiplies by up to 2^24 / 1e-20 * quantum, which has to stay finite).

@@ -293,25 +293,17 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
   //   stack(n) = [n has two inner children] + [a slot of n is no inner child] + max stack(inner child).
   // An entry that waits keeps its place while children of it are visited, which
   // the sum covers.  Children are numbered after their parents.
-  std::vector<uint32_t> stack(out->nodes.size(), 0), pending(out->nodes.size(), 0), depth(out->nodes.size(), 1);
+  std::vector<uint32_t> stack(out->nodes.size(), 0), depth(out->nodes.size(), 1);
   for (size_t i = out->nodes.size(); i-- > 0;) {
     const WideNodeHost& n = out->nodes[i];
     const uint32_t numInner = (uint32_t)__builtin_popcount(n.exps >> 24);
-    uint32_t leaves = 0, end = 0;
-    for (int s = 0; s < W; ++s) {
-      leaves += n.ends[s] > end ? 1 : 0;
-      end = n.ends[s];
-    }
     for (uint32_t c = n.firstChild; c < n.firstChild + numInner; ++c) {
       stack[i] = std::max(stack[i], stack[c]);
-      pending[i] = std::max(pending[i], pending[c]);
       depth[i] = std::max(depth[i], depth[c] + 1);
     }
     stack[i] += (numInner > 1 ? 1 : 0) + (numInner < (uint32_t)W ? 1 : 0);
-    pending[i] += numInner + leaves - (numInner > 0 ? 1 : 0);
   }
   out->maxStack = stack[0];
-  out->maxPending = pending[0];
   out->depth = depth[0];
   return std::string();
 }

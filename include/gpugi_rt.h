@@ -411,9 +411,9 @@ int gpugi_trace(gpugi_ctx* ctx, int query, int kernel, const gpugi_ray* rays, gp
  * a triangle pass instead of a box pass.  Default (2, 10, 8, 8): the fastest
  * incoherent closest-hit configuration on the 2,097,152-triangle heightfield.  No
  * reference counterpart: the GLSL path has one fixed layout
- * (TRIANGLES_PER_LEAF, scenedata.glsl:5).  A stack entry holds the children of
- * one node that wait; gpugi_get_wide_config's max_stack is the most children
- * that can wait on one ray's stack in the loaded scene. */
+ * (TRIANGLES_PER_LEAF, scenedata.glsl:5).  gpugi_get_wide_config's
+ * max_stack is the most stack entries that a ray can need in the loaded scene
+ * (an entry holds the children of one node that wait). */
 int gpugi_set_wide_config(gpugi_ctx* ctx, int max_leaf_triangles, int lds_stack_entries, int refill_lanes,
                           int wait_lanes);
 int gpugi_get_wide_config(gpugi_ctx* ctx, int* max_leaf_triangles, int* lds_stack_entries, int* refill_lanes,

@@ -76,10 +76,10 @@ void TraceS(bool any, bool wt, const WideScene& s, const float* rays, int32_t* h
 }  // namespace
 
 // Traces n rays (8 floats each) into hits (4 words each).  counts: {nodes, triangles,
-// max pending, max stack entries, entries the deepest ray used, overflow flag, nodes visited}.
+// max stack entries, entries the deepest ray used, overflow flag, nodes visited}.
 // ldsEntries: 1 or 10.  Returns 0, or 1 if the tree could not be built.
 extern "C" int wide_walk(const gpugi_scene_desc* d, uint32_t leaf, int any, int wt, int ldsEntries, const float* rays,
-                         int32_t* hits, size_t n, uint32_t counts[7]) {
+                         int32_t* hits, size_t n, uint32_t counts[6]) {
   WideBVHHost b;
   if (!BuildWideBVH(*d, leaf, &b, wt != 0).empty()) return 1;
   uint32_t flag = 0;
@@ -96,12 +96,11 @@ extern "C" int wide_walk(const gpugi_scene_desc* d, uint32_t leaf, int any, int 
   else TraceS<10>(any != 0, wt != 0, s, rays, hits, n, &lds, &spill);
   counts[0] = (uint32_t)b.nodes.size();
   counts[1] = (uint32_t)b.tris.size();
-  counts[2] = b.maxPending;
-  counts[3] = b.maxStack;
-  counts[4] = 0;
-  for (int e = 0; e < ldsEntries; ++e) counts[4] += lds[(size_t)e * kLanes + 1].x != 0xdeadu;
-  for (const uint2& e : spill) counts[4] += e.x != 0xdeadu;
-  counts[5] = flag;
-  counts[6] = slots_tested / kWideArity;
+  counts[2] = b.maxStack;
+  counts[3] = 0;
+  for (int e = 0; e < ldsEntries; ++e) counts[3] += lds[(size_t)e * kLanes + 1].x != 0xdeadu;
+  for (const uint2& e : spill) counts[3] += e.x != 0xdeadu;
+  counts[4] = flag;
+  counts[5] = slots_tested / kWideArity;
   return 0;
 }

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from gpugi_amd import workloads
+from test_wide_walk_cpu import centre_camera, nested_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -68,14 +69,16 @@ def test_batch_stack_depths_match_single_scene(rt, ctx, stack):
     """The LDS stack depth of the wide walk (16, 24 or 32 entries per lane;
     deeper entries spill to global memory) changes where the traversal stack
     lives, not what it holds: every depth gives the single-scene image bit for
-    bit.  The 24-cell heightfield needs 19 entries (in LDS from depth 24 on),
-    the 30-sphere clutter room 36 (it spills at every depth)."""
+    bit.  The 30-sphere clutter room needs up to 12 entries (always in LDS); the
+    nested quads' camera rays need over 32 (they spill at every depth)."""
     scenes = small_scenes(rt)
     hs = rt.HostScene.clutter(30, 5)
     scenes.append((hs, workloads.clutter_camera(32, 32), 32, 32, rt.LightSampler(hs, 7).generate(128)))
+    hs = nested_scene(60)
+    hs.add_point_light((0.9, 0.8, 1.1), (1.0, 1.0, 1.0))
+    scenes.append((hs, centre_camera(64), 64, 64, rt.LightSampler(hs, 3).generate(128)))
     ctx.load_scene(hs)
-    ctx.set_wide_config(2, 16, 8, 16)
-    assert ctx.wide_config()["max_stack"] > 32  # the spill path is exercised at every depth
+    assert ctx.wide_config()["max_stack"] > 90
     b = rt.Batch(0)
     try:
         for hs, cam, w, h, lights in scenes:
@@ -93,7 +96,6 @@ def test_batch_stack_depths_match_single_scene(rt, ctx, stack):
         with pytest.raises(rt.GpugiError):
             b.config(rt.KERNEL_WIDE, 2, 2, 20)
     finally:
-        ctx.set_wide_config(2, 10, 8, 16)
         b.close()
 
 

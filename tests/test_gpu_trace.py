@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from gpugi_amd import workloads
+from test_wide_walk_cpu import centre_rays, nested_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -169,9 +170,10 @@ def test_full_size_incoherent_set_properties(rt, oracle, ctx):
 
 @pytest.mark.parametrize("leaf,stack,refill,wait", [(1, 4, 64, 1), (8, 4, 1, 64), (2, 24, 16, 32), (4, 8, 8, 16)])
 def test_wide_configurations(rt, oracle, ctx, leaf, stack, refill, wait):
-    """Every wide configuration gives the same answers: a 4-entry LDS stack
-    spills to global memory on most rays, wait 1 runs a leaf pass as soon as a
-    lane waits, wait 64 only when no lane can traverse."""
+    """Every wide configuration gives the same answers: wait 1 runs a leaf pass as
+    soon as a lane waits, wait 64 only when no lane can traverse.  Most rays to
+    the nested quads' centre need more than 24 stack entries: every configuration
+    spills to global memory on them."""
     print("case: wide config", leaf, stack, refill, wait, flush=True)
     hs = rt.HostScene.heightfield(64, workloads.MASTER_SEED)
     ctx.load_scene(hs)
@@ -180,8 +182,6 @@ def test_wide_configurations(rt, oracle, ctx, leaf, stack, refill, wait):
     cfg = ctx.wide_config()
     assert (cfg["max_leaf_triangles"], cfg["lds_stack_entries"], cfg["refill_lanes"], cfg["wait_lanes"]) == \
         (leaf, stack, refill, wait)
-    if stack == 4:
-        assert cfg["max_stack"] > stack  # the spill path is exercised
     for rays in (prim, diff):
         want = oracle.trace(sc, rays)
         got = hits_int(ctx.trace(rays_struct(rt, rays), rt.CLOSEST_HIT, rt.KERNEL_WIDE))
@@ -190,6 +190,14 @@ def test_wide_configurations(rt, oracle, ctx, leaf, stack, refill, wait):
     want_any = oracle.trace(sc, shadow, any_hit=True)[:, 0]
     got_any = hits_int(ctx.trace(rays_struct(rt, shadow), rt.ANY_HIT, rt.KERNEL_WIDE))[:, 0]
     assert (got_any != want_any).sum() <= max(2, 1e-3 * len(shadow))
+    hs = nested_scene(60)
+    ctx.load_scene(hs)
+    assert ctx.wide_config()["max_stack"] > 90
+    sc, rays = oracle.Scene(hs.arrays()), centre_rays(5001, 9)
+    got = hits_int(ctx.trace(rays_struct(rt, rays), rt.CLOSEST_HIT, rt.KERNEL_WIDE))
+    assert np.array_equal(got, oracle.bruteforce(sc, rays))
+    got_any = hits_int(ctx.trace(rays_struct(rt, rays), rt.ANY_HIT, rt.KERNEL_WIDE))[:, 0]
+    assert np.array_equal(got_any, oracle.bruteforce(sc, rays, any_hit=True)[:, 0])
     ctx.set_wide_config(2, 10, 8, 16)
 
 

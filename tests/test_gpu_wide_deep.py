@@ -3,7 +3,7 @@ their LDS part (test_wide_walk_cpu.py's nested quads: over 48 entries)."""
 import numpy as np
 import pytest
 
-from test_wide_walk_cpu import centre_rays, nested_scene
+from test_wide_walk_cpu import centre_camera, centre_rays, nested_scene, walk  # noqa: F401 (walk is a fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -26,12 +26,26 @@ def test_trace_spills_on_a_deep_tree(rt, oracle, ctx, stack):
         ctx.set_wide_config(2, 10, 8, 16)
 
 
+def test_max_stack_is_the_walks_bound(rt, walk, ctx):  # noqa: F811
+    """gpugi_get_wide_config's max_stack: the stack entries the walk is given, not the children in them."""
+    for hs, leaf in ((nested_scene(60), 1), (rt.HostScene.heightfield(64, 5), 2), (rt.HostScene.cornell(), 8)):
+        ctx.load_scene(hs)
+        default = ctx.wide_config()
+        ctx.set_wide_config(leaf, 10)
+        try:
+            _, n = walk(hs, centre_rays(1, 1), leaf)
+            assert ctx.wide_config()["max_stack"] == n["stack"]
+        finally:
+            ctx.set_wide_config(*(default[k] for k in ("max_leaf_triangles", "lds_stack_entries", "refill_lanes",
+                                                       "wait_lanes")))
+
+
 def test_path_tracer_spills_on_a_deep_tree(rt, ctx):
     """The path tracer's 16 entries and the batch's 16, 24 and 32 give one image: where the stack lives
     does not change it."""
     hs = nested_scene(60)
     hs.add_point_light((0.9, 0.8, 1.1), (1.0, 1.0, 1.0))
-    cam = rt.camera((1.3, 1.2, 1.1), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 20.0, 64, 64)
+    cam = centre_camera(64)
     lights = rt.LightSampler(hs, 3).generate(128)
     ctx.load_scene(hs)
     ctx.set_screen(64, 64)

@@ -29,12 +29,12 @@ def walk(tmp_path_factory):
 
     def run(scene, rays, leaf=2, any_hit=False, watertight=False, lds=10):
         rays = np.ascontiguousarray(rays, np.float32)
-        hits, counts = np.zeros((len(rays), 4), np.int32), np.zeros(7, np.uint32)
+        hits, counts = np.zeros((len(rays), 4), np.int32), np.zeros(6, np.uint32)
         p = ctypes.c_void_p
         assert fn(ctypes.byref(scene.desc()), ctypes.c_uint32(leaf), int(any_hit), int(watertight), lds,
                   p(rays.ctypes.data), p(hits.ctypes.data), ctypes.c_size_t(len(rays)), p(counts.ctypes.data)) == 0
-        assert counts[5] == 0 and counts[4] <= counts[3]  # no overflow, the stack bound holds
-        return hits, dict(zip(("nodes", "tris", "pending", "stack", "used", "flag", "visits"), counts.tolist()))
+        assert counts[4] == 0 and counts[3] <= counts[2]  # no overflow, the stack bound holds
+        return hits, dict(zip(("nodes", "tris", "stack", "used", "flag", "visits"), counts.tolist()))
     return run
 
 
@@ -162,6 +162,12 @@ def five_ary_chain(levels, seed):
     return TreeScene(node)
 
 
+def centre_camera(size):
+    """A camera whose every ray passes so close to the nested quads' centre that its walk has over 32 stack
+    entries at a time (test_deep_tree_uses_the_spill_stack)."""
+    return _rt.camera((1.3, 1.2, 1.1), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 1e-5, size, size)
+
+
 SCENES = {"cornell": _rt.HostScene.cornell, "heightfield": lambda: _rt.HostScene.heightfield(20, 7),
           "clutter": lambda: _rt.HostScene.clutter(3, 5), "nested": lambda: nested_scene(30),
           "triangle": lambda: _rt.HostScene.build([[0, 0, 0], [1, 0, 0.2], [0, 1, 0.1]], [[0, 1, 2]])}
@@ -201,6 +207,8 @@ def test_deep_tree_uses_the_spill_stack(walk, oracle):
     assert n["used"] > 48
     got, n = walk(hs, rays, 1, any_hit=True, lds=10)
     assert np.array_equal(got[:, 0], oracle.bruteforce(sc, rays, any_hit=True)[:, 0])
+    for ray in oracle.raygen_primary(centre_camera(64), 64, 64, 1, 4096)[::97]:
+        assert walk(hs, ray[None], 2, lds=10)[1]["used"] > 32
 
 
 @pytest.mark.parametrize("distance", [3e5, 3e6, 1e7])
