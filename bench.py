@@ -467,7 +467,7 @@ def clutter_sweep():
     R = workloads.SceneRays(ctx, workloads.clutter_camera(workloads.HF_WIDTH, workloads.HF_HEIGHT),
                             workloads.CLUTTER_LIGHTS, n, workloads.MASTER_SEED, workloads.HF_WIDTH,
                             workloads.HF_HEIGHT)
-    sweep_wide_configs(ctx, R, n, itertools.product((2, 4), (8, 10, 12, 16, 24), (8, 16), (16, 24)))
+    sweep_wide_configs(ctx, R, n, itertools.product((2, 4), (8, 10, 12, 16, 24), (8, 16), (8, 16, 24)))
     R.free()
     ctx.close()
 

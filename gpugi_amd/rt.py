@@ -672,7 +672,7 @@ class Context:
         self._call("gpugi_trace_noalloc", int(query), int(kernel), ctypes.c_void_p(rays_buf.ptr),
                    ctypes.c_void_p(hits_buf.ptr), ctypes.c_size_t(n))
 
-    def set_wide_config(self, max_leaf_triangles, lds_stack_entries, refill_lanes=8, wait_lanes=16):
+    def set_wide_config(self, max_leaf_triangles, lds_stack_entries, refill_lanes=8, wait_lanes=8):
         self._call("gpugi_set_wide_config", int(max_leaf_triangles), int(lds_stack_entries), int(refill_lanes),
                    int(wait_lanes))
 
@@ -832,7 +832,7 @@ class Batch:
     def finalize(self):
         self._call("gpugi_batch_finalize")
 
-    def config(self, kernel=KERNEL_WIDE, tiles_per_grab=2, grid_multiplier=2, stack_depth=16):
+    def config(self, kernel=KERNEL_WIDE, tiles_per_grab=2, grid_multiplier=4, stack_depth=16):
         self._call("gpugi_batch_config", int(kernel), int(tiles_per_grab), int(grid_multiplier), int(stack_depth))
 
     def reset(self, frame_index=0):

@@ -198,14 +198,25 @@ def test_wide_configurations(rt, oracle, ctx, leaf, stack, refill, wait):
     assert np.array_equal(got, oracle.bruteforce(sc, rays))
     got_any = hits_int(ctx.trace(rays_struct(rt, rays), rt.ANY_HIT, rt.KERNEL_WIDE))[:, 0]
     assert np.array_equal(got_any, oracle.bruteforce(sc, rays, any_hit=True)[:, 0])
-    ctx.set_wide_config(2, 10, 8, 16)
+    ctx.set_wide_config(2, 10)
+
+
+def test_binding_defaults_are_the_shipped_configuration(rt):
+    c = rt.Context(0)
+    try:
+        shipped = c.wide_config()
+        assert shipped["wait_lanes"] == 8
+        c.set_wide_config(shipped["max_leaf_triangles"], shipped["lds_stack_entries"])
+        assert c.wide_config() == shipped
+    finally:
+        c.close()
 
 
 @pytest.mark.parametrize("query", ["closest", "any"])
 def test_autotune_trace_keeps_answers(rt, oracle, ctx, query):
     """gpugi_autotune_trace searches leaf size, LDS stack depth, refill and
     wait thresholds on the given rays and keeps the fastest; the default
-    configuration (leaf 2, stack 10, refill 8, wait 16) is one of the timed
+    configuration (leaf 2, stack 10, refill 8, wait 8) is one of the timed
     points, so the result is never slower than it on those rays.  After the
     search the scene's wide BVH is rebuilt for the chosen leaf size and the
     wide kernel must still give the oracle's answers."""
@@ -234,7 +245,7 @@ def test_autotune_trace_keeps_answers(rt, oracle, ctx, query):
             want = oracle.trace(sc, rays, any_hit=True)[:, 0]
             assert (got[:, 0] != want).sum() <= max(2, 1e-3 * n)
     finally:
-        ctx.set_wide_config(2, 10, 8, 16)
+        ctx.set_wide_config(2, 10)
 
 
 @pytest.mark.parametrize("scene", ["heightfield", "clutter"])

@@ -13,7 +13,7 @@ def test_trace_spills_on_a_deep_tree(rt, oracle, ctx, stack):
     hs = nested_scene(60)
     sc, rays = oracle.Scene(hs.arrays()), centre_rays(20001, 9)
     ctx.load_scene(hs)
-    ctx.set_wide_config(1, stack, 8, 16)
+    ctx.set_wide_config(1, stack)
     try:
         print("case: deep tree, %d LDS entries" % stack, flush=True)
         r = rays.view(rt.RAY_DTYPE).reshape(-1)
@@ -23,21 +23,19 @@ def test_trace_spills_on_a_deep_tree(rt, oracle, ctx, stack):
         want = oracle.bruteforce(sc, rays, any_hit=True)[:, 0]
         assert 0 < want.sum() < len(want) and np.array_equal(got, want)
     finally:
-        ctx.set_wide_config(2, 10, 8, 16)
+        ctx.set_wide_config(2, 10)
 
 
 def test_max_stack_is_the_walks_bound(rt, walk, ctx):  # noqa: F811
     """gpugi_get_wide_config's max_stack: the stack entries the walk is given, not the children in them."""
     for hs, leaf in ((nested_scene(60), 1), (rt.HostScene.heightfield(64, 5), 2), (rt.HostScene.cornell(), 8)):
         ctx.load_scene(hs)
-        default = ctx.wide_config()
         ctx.set_wide_config(leaf, 10)
         try:
             _, n = walk(hs, centre_rays(1, 1), leaf)
             assert ctx.wide_config()["max_stack"] == n["stack"]
         finally:
-            ctx.set_wide_config(*(default[k] for k in ("max_leaf_triangles", "lds_stack_entries", "refill_lanes",
-                                                       "wait_lanes")))
+            ctx.set_wide_config(2, 10)
 
 
 def test_path_tracer_spills_on_a_deep_tree(rt, ctx):
