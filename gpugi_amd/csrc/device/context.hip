@@ -177,6 +177,7 @@ RefScene MakeRef(const gpugi_ctx* c) {
   s.positions = (const float*)c->dPos;
   s.vinfo = (const float4*)c->dVinfo;
   s.obox = c->sceneObox ? 1 : 0;
+  s.numNodes = c->numNodes;
   return s;
 }
 

@@ -14,42 +14,58 @@ namespace gpugi {
 // steps of every lane without a leaf to test, or, once a quarter of the lanes at
 // work have one, a leaf step of those.  A ray waits at its leaf, since its next
 // box test needs the leaf's hit distance.  Lanes whose ray has ended take the
-// next rays of the wave's batches once kRefRefill are idle.
+// next rays of the wave's batches once kRefRefill are idle; but where every wave has
+// several batches and the rays of the one at hand all point into one octant, only
+// once all have ended: such rays mostly end together, and a refill stalls the wave
+// for the new rays' load (2^23 camera rays, room of 16 spheres: 740 -> 660 us).
 // Bound by the dependent 32-byte node loads.  With one thread per ray almost every
 // turn of a wave's loop ran the triangle test for a few lanes, and a wave lasted
 // as long as its longest ray: 2^20 diffuse rays on a 524,288-triangle
 // heightfield 866 -> 472 us, 2^24 on the 2,097,152-triangle one 13.0 -> 6.2 ms
 // (2.7 Grays/s).  A leaf step at an eighth of the lanes: 492 us; at 16 lanes: 593 us;
-// two box steps a turn: 635 us against 593 with four.
-// Waves are dealt out statically (the walk needs no memory but the caller's):
-// block b runs on XCD b % 8, XCD x owns the x-th eighth of the ray array and its
-// waves take that eighth's 64-ray batches in turn.
-constexpr int kRefRefill = 8, kRefBoxSteps = 4;
-constexpr uint32_t kRefXcds = 8, kRefWaves = 256 / 64;
+// two box steps a turn: 635 us against 593 with four.  Refills at 8 idle lanes: 2.66
+// against 2.50 ms for 2^23 diffuse rays on the 524,288-triangle heightfield.
+// Waves are dealt out statically (the walk needs no memory but the caller's): block
+// b runs on XCD b % 8, and the waves of an XCD take its batches in turn.  XCD x's
+// are the x-th eighth of the ray array, so that neighbouring rays share an L2; from
+// four batches a wave on it has every eighth chunk of 2^kRefChunkLog2 batches, since
+// the eighths of an image can cost very differently, and the launch waits for the
+// dearest (2^21 camera rays, room of 400 spheres: 1230 -> 950 us; the larger the
+// chunks, the less so: 2^23 camera rays, 524,288-triangle heightfield, 1.57 ms with
+// 2^8 batches, 1.85 with 2^10).
+constexpr int kRefBoxSteps = 4;
+constexpr uint32_t kRefRefill = 16, kRefXcds = 8, kRefWaves = 256 / 64, kRefChunkLog2 = 8;
+constexpr uint32_t kRefTinyNodes = 1024, kRefL2Nodes = (4u << 20) / 32;
 
 template <bool ANY, bool WT, bool OBOX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_trace_ref(
     RefScene s, const float4* __restrict__ rays, int4* __restrict__ hits, uint32_t n,
-    const uint32_t* __restrict__ nDev) {
+    const uint32_t* __restrict__ nDev, uint32_t resident) {
   if (nDev) n = min(*nDev, n);  // the ray count as the device holds it
   const int lane = threadIdx.x & 63;
   const uint64_t below = (1ull << lane) - 1ull;
-  const uint32_t batches = (n + 63u) / 64u, perX = (batches + kRefXcds - 1) / kRefXcds;
-  const uint32_t bEnd = min(batches, (blockIdx.x % kRefXcds + 1) * perX);
+  const uint32_t batches = (n + 63u) / 64u, perX = (batches + kRefXcds - 1u) / kRefXcds;
+  const uint32_t xcd = blockIdx.x % kRefXcds;
   const uint32_t stride = gridDim.x / kRefXcds * kRefWaves;
-  // wave-uniform: the next batch, the batch being handed out and how many of its rays are gone
-  uint32_t nextBatch = blockIdx.x % kRefXcds * perX + blockIdx.x / kRefXcds * kRefWaves +
+  const bool several = batches >= 2u * resident;
+  const bool inChunks = several && (s.numNodes <= kRefTinyNodes || batches >= 4u * resident);
+  constexpr uint32_t mask = (1u << kRefChunkLog2) - 1u;
+  // wave-uniform: which of the XCD's batches is next, the batch being handed out, how
+  // many of its rays are gone, and the idle lanes to wait for
+  uint32_t nextOfXcd = blockIdx.x / kRefXcds * kRefWaves +
                        (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
-  uint32_t cur = 0, pos = 64;
+  uint32_t cur = 0, pos = 64, refill = kRefRefill;
   bool exhausted = false, active = false;
   uint32_t ri = 0;
   RefWalk w;
   for (;;) {
     const uint64_t idle = ~__ballot(active);
     const uint32_t nidle = (uint32_t)__popcll(idle);
-    if (!exhausted && nidle >= (uint32_t)kRefRefill) {
-      const uint32_t avail = 64u - pos, next = nextBatch;
-      const bool more = avail < nidle && next < bEnd;
+    if (!exhausted && nidle >= refill) {
+      const uint32_t avail = 64u - pos;
+      const uint32_t next = inChunks ? (nextOfXcd & ~mask) * kRefXcds + (xcd << kRefChunkLog2) + (nextOfXcd & mask)
+                                     : xcd * perX + nextOfXcd;
+      const bool more = avail < nidle && next < batches && (inChunks || nextOfXcd < perX);
       if (!active) {
         const uint32_t rank = (uint32_t)__popcll(idle & below);
         uint32_t r = n;
@@ -67,9 +83,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
       } else if (more) {
         cur = next;
         pos = nidle - avail;
-        nextBatch += stride;
+        nextOfXcd += stride;
       } else {
         exhausted = true;
+      }
+      if (several && nidle == 64u) {
+        const uint64_t all = __ballot(active), x = __ballot(active && w.d.x < 0.0f),
+                       y = __ballot(active && w.d.y < 0.0f), z = __ballot(active && w.d.z < 0.0f);
+        refill = (x == 0 || x == all) && (y == 0 || y == all) && (z == 0 || z == all) ? 64u : kRefRefill;
       }
     }
     const uint64_t act = __ballot(active);
@@ -158,22 +179,27 @@ hipError_t LaunchTraceRef(const RefScene& s, int query, const gpugi_ray* rays, g
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess) return e;
-  // A wave for every batch, at most eight blocks per CU, which hide the loads'
-  // latency best, or four where each still gets eight batches and more, which share
-  // the L1 better (2^24 rays: 6.2 against 6.8 ms; 2^20: 506 against 492 us); whole
-  // blocks per XCD.
-  const size_t perX = ((n + 63) / 64 + kRefXcds - 1) / kRefXcds;
-  const size_t perCu = perX * kRefXcds >= (size_t)cus * 4 * kRefWaves * 8 ? 4 : 8;
-  const size_t most = std::max<size_t>(1, (size_t)cus * perCu / kRefXcds);
-  dim3 grid((unsigned)(kRefXcds * std::min((perX + kRefWaves - 1) / kRefWaves, most)));
-  typedef void (*Kernel)(RefScene, const float4*, int4*, uint32_t, const uint32_t*);
+  // A wave for every batch on a tree of some dozen triangles: its rays end after a few
+  // steps, and waves that the hardware deals out balance better than refills pay
+  // (Cornell room, 2^21 camera / diffuse / shadow rays: 71 / 234 / 127 us; 94 / 239 / 158
+  // with resident waves).  Else at most eight blocks per CU, which hide the loads'
+  // latency best, or six where each still gets four batches and more and the tree is
+  // larger than an XCD's L2 (4 MB): fewer waves share the L1 better (2^23 diffuse rays,
+  // 2,097,152-triangle heightfield: 3.1 against 3.4 ms).  Whole blocks per XCD.
+  const uint32_t batches = (uint32_t)((n + 63) / 64);
+  const uint32_t perX = (batches + kRefXcds - 1) / kRefXcds;
+  const uint32_t resident = (uint32_t)cus * 8 * kRefWaves, blocks = (perX + kRefWaves - 1) / kRefWaves;
+  const uint32_t perCu = batches >= 4 * resident && s.numNodes > kRefL2Nodes ? 6 : 8;
+  const uint32_t most = s.numNodes <= kRefTinyNodes ? blocks : std::max(1u, (uint32_t)cus * perCu / kRefXcds);
+  dim3 grid(kRefXcds * std::min(blocks, most));
+  typedef void (*Kernel)(RefScene, const float4*, int4*, uint32_t, const uint32_t*, uint32_t);
   static const Kernel kernels[2][2][2] = {
       {{k_trace_ref<false, false, false>, k_trace_ref<false, false, true>},
        {k_trace_ref<false, true, false>, k_trace_ref<false, true, true>}},
       {{k_trace_ref<true, false, false>, k_trace_ref<true, false, true>},
        {k_trace_ref<true, true, false>, k_trace_ref<true, true, true>}}};
   const Kernel fn = kernels[query == GPUGI_ANY_HIT][watertight ? 1 : 0][s.obox ? 1 : 0];
-  hipLaunchKernelGGL(fn, grid, dim3(256), 0, stream, s, (const float4*)rays, (int4*)hits, (uint32_t)n, nDevice);
+  hipLaunchKernelGGL(fn, grid, dim3(256), 0, stream, s, (const float4*)rays, (int4*)hits, (uint32_t)n, nDevice, resident);
   return hipGetLastError();
 }
 

@@ -17,6 +17,7 @@ struct RefScene {
   const float* __restrict__ positions;  // VertexPositionBuffer RGB32F, TBO 2
   const float4* __restrict__ vinfo;     // VertexInfoBuffer, TBO 3
   int obox = 0;                         // nodes are TreeNode<OBox>: 3 texels each (OBOX_BVH)
+  uint32_t numNodes = 0;
 };
 
 // TRACERAY_IMPORTANCE_BREAK (traceray.glsl:48-112): per-node importance {x, y}
