@@ -53,7 +53,7 @@ struct gpugi_ctx {
   void* dWideQueue = nullptr;  // the wide trace kernel's batch counters
   size_t spillBytes = 0;
   uint32_t wideMaxStack = 0, wideNumNodes = 0;
-  float wideTScale = 1.0f;
+  float wideTScale = 1.0f, wideCrossings = 0.0f;
   std::map<int, int> wideBlocksPerCU;  // per LDS stack depth: resident blocks of the trace kernel
   int wideLeaf = 2;     // triangles per merged wide leaf
   int wideStack = 10;   // LDS stack entries per lane of the trace kernel
@@ -278,6 +278,7 @@ int RebuildWide(gpugi_ctx* ctx) {
                            hipMemcpyHostToDevice));
   ctx->wideMaxStack = wide.maxStack;
   ctx->wideTScale = wide.tScale;
+  ctx->wideCrossings = wide.crossings;
   ctx->wideNumNodes = (uint32_t)wide.nodes.size();
   ctx->hasWide = true;
   return GPUGI_OK;
@@ -778,6 +779,7 @@ static DrawParams MakeDrawParams(gpugi_ctx* ctx, uint32_t frame_seed) {
   p.wide = MakeWide(ctx, kWideLdsStack);
   p.useWide = ctx->hasWide && ctx->integratorKernel != GPUGI_KERNEL_REFERENCE;
   p.wideNodes = ctx->wideNumNodes;
+  p.wideCrossings = ctx->wideCrossings;
   p.materials = (const gpugi_material*)ctx->dMats;
   p.lights = (const gpugi_light_sample*)ctx->dLights;
   p.numLights = ctx->numLights;

@@ -17,6 +17,7 @@ struct DrawParams {
   WideScene wide;
   bool useWide = false;
   uint32_t wideNodes = 0;                 // nodes of the wide BVH
+  float wideCrossings = 0.0f;             // WideBVHHost::crossings
   const gpugi_material* materials = nullptr;
   const gpugi_light_sample* lights = nullptr;
   uint32_t numLights = 0;
@@ -88,16 +89,24 @@ struct IntegratorState {
 constexpr uint32_t kPhasedMinLanes = 16;
 hipError_t PersistentGrid(IntegratorState* st, const void* kernel, size_t items, uint32_t* blocks,
                           hipStream_t stream, bool resident = true, uint32_t* lanes = nullptr);
-// Whether the paths of `items` pixels stay in step: at most one wave per SIMD
-// (no lane gets a second pixel) in a tree of at most kInStepNodes nodes, whose
-// rays all end after a few passes.  Such images are faster with each ray traced
-// where it is needed than in phases: 220 against 251 us a frame in the Cornell
-// room, 203 against 223 on a 64 x 64 heightfield (1,000 nodes), both 256 x 256
-// pixels; with 2,600 nodes (room of 16 spheres) phases win, 260 against 280, and
-// so they do in the Cornell room at 1024 x 1024, 704 against 729.
-constexpr uint32_t kInStepNodes = 1536;
+// Whether `items` paths stay in step, so that tracing each ray where it is needed
+// is faster than phases: at most kInStepWaves waves per SIMD (hardly a lane gets a
+// second path), and either a tree of at most kInStepNodes nodes, whose rays all end
+// after a few passes, or light paths in an open scene (fewer than kOpenCrossings),
+// most of which leave it at once.  Time in phases over time in step (path length 5):
+//                                       256x256 512x512 640x640 768x768 pixels
+//   path tracer, Cornell room (5 nodes)    1.22    1.17    1.00    0.95
+//     64 x 64 heightfield (822 nodes)      1.11    1.14    1.07    1.12
+//     room of 16 spheres (2,452)           0.94    0.99    0.92    0.86
+//   light tracer, Cornell room             1.17    1.26    1.20    1.05
+//     64 x 64 heightfield                  1.44    1.27    1.08    0.93
+//     1024 x 1024 heightfield (221,288)    1.22    1.23    1.09    1.00
+//     room of 16 spheres                   0.96    0.99    0.85    0.82
+//     room of 400 spheres (61,488)         0.83    0.86       -    0.75
+constexpr uint32_t kInStepNodes = 1536, kInStepWaves = 7;
+constexpr float kOpenCrossings = 1.5f;
 hipError_t EnsureSimds(IntegratorState* st);
-bool PathsInStep(const IntegratorState* st, const DrawParams& p, size_t items);
+bool PathsInStep(const IntegratorState* st, const DrawParams& p, size_t items, bool light);
 
 // Grows a device buffer to at least `bytes` (contents are not preserved).
 inline hipError_t EnsureBuffer(void** buf, size_t* cap, size_t bytes) {

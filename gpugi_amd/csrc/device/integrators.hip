@@ -71,8 +71,9 @@ hipError_t EnsureSimds(IntegratorState* st) {
   return e;
 }
 
-bool PathsInStep(const IntegratorState* st, const DrawParams& p, size_t items) {
-  return p.wideNodes <= kInStepNodes && items <= (size_t)st->simds * kTileThreads;
+bool PathsInStep(const IntegratorState* st, const DrawParams& p, size_t items, bool light) {
+  return items <= (size_t)st->simds * kTileThreads * kInStepWaves &&
+         (p.wideNodes <= kInStepNodes || (light && p.wideCrossings < kOpenCrossings));
 }
 
 hipError_t PersistentGrid(IntegratorState* st, const void* kernel, size_t items, uint32_t* blocks,
@@ -106,7 +107,7 @@ static hipError_t DrawPT(IntegratorState* st, const DrawParams& p0, hipStream_t 
   if (tiles == 0) return hipSuccess;
   typedef void (*Kernel)(DrawParams, uint32_t*, uint32_t);
   if (hipError_t e = EnsureSimds(st)) return e;
-  const bool phased = p.useWide && !PathsInStep(st, p, tiles * kTileThreads);
+  const bool phased = p.useWide && !PathsInStep(st, p, tiles * kTileThreads, false);
   const Kernel fn = phased ? (p.watertight ? k_pathtracer_wide<true> : k_pathtracer_wide<false>)
                            : (p.useWide ? k_pathtracer<true> : k_pathtracer<false>);
   uint32_t blocks = 0, lanes = kTileThreads;

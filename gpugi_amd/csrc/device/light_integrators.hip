@@ -520,7 +520,7 @@ static hipError_t LaunchLight(IntegratorState* st, const DrawParams& p, int R, u
   typedef void (*Kernel)(DrawParams, int, uint32_t, LightCacheEntryDev*, LightCacheEntryDev*, uint32_t*, uint32_t*,
                          uint32_t);
   if (hipError_t e = EnsureSimds(st)) return e;
-  const bool phased = p.useWide && !PathsInStep(st, p, paths);
+  const bool phased = p.useWide && !PathsInStep(st, p, paths, true);
   const Kernel fn = phased ? (p.watertight ? k_lighttracer_wide<MODE, true> : k_lighttracer_wide<MODE, false>)
                            : (p.useWide ? k_lighttracer<true, MODE> : k_lighttracer<false, MODE>);
   uint32_t blocks = 0, lanes = kLightBlock;
@@ -624,7 +624,7 @@ hipError_t DrawBPT(IntegratorState* st, const DrawParams& p0, hipStream_t stream
   const size_t pixels = (size_t)(p.width / kTile) * (p.height / kTile) * kTileThreads;
   if (pixels) {
     typedef void (*Kernel)(DrawParams, const LightCacheEntryDev*, const uint32_t*, uint32_t*, uint32_t);
-    const bool phased = p.useWide && !PathsInStep(st, p, pixels);
+    const bool phased = p.useWide && !PathsInStep(st, p, pixels, false);
     const Kernel fn = phased ? (p.watertight ? k_bpt_eye_wide<true> : k_bpt_eye_wide<false>)
                              : (p.useWide ? k_bpt_eye<true> : k_bpt_eye<false>);
     uint32_t blocks = 0, lanes = kTileThreads;

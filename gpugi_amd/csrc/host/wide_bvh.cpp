@@ -62,6 +62,7 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
   kidsAt[v.n] = (uint32_t)kids.size();
   // Subtree valid-triangle counts, bottom-up (children follow parents in preorder).
   std::vector<uint32_t> count(v.n, 0);
+  double area = 0.0;  // twice the triangles'
   for (uint32_t ii = v.n; ii-- > 0;) {
     uint32_t c = 0;
     if (v.isLeafNode(ii)) {
@@ -71,12 +72,25 @@ std::string BuildWideBVH(const gpugi_scene_desc& desc, uint32_t maxLeafTris, Wid
         const int32_t* t = desc.triangles + ((size_t)leaf * tpl + k) * 4;
         if (t[0] == t[1]) break;
         ++c;
+        double e0[3], e1[3], n2 = 0.0;
+        for (int a = 0; a < 3; ++a) {
+          const double p0 = desc.positions[(size_t)t[0] * 3 + a];
+          e0[a] = desc.positions[(size_t)t[1] * 3 + a] - p0;
+          e1[a] = desc.positions[(size_t)t[2] * 3 + a] - p0;
+        }
+        for (int a = 0; a < 3; ++a) {
+          const int b = (a + 1) % 3, d = (a + 2) % 3;
+          const double x = e0[b] * e1[d] - e0[d] * e1[b];
+          n2 += x * x;
+        }
+        area += std::sqrt(n2);
       }
     } else {
       for (uint32_t k = kidsAt[ii]; k < kidsAt[ii + 1]; ++k) c += count[kids[k]];
     }
     count[ii] = c;
   }
+  out->crossings = v.surface(0) > 0.0f ? (float)(area / (double)v.surface(0)) : 0.0f;
   out->nodes.clear();
   out->tris.clear();
   out->tris.reserve(count[0]);
