@@ -99,6 +99,27 @@ def test_batch_stack_depths_match_single_scene(rt, ctx, stack):
         b.close()
 
 
+@pytest.mark.parametrize("scenes", [5, 6])
+def test_batch_at_the_edge_of_staying_in_step(rt, ctx, scenes):
+    """Five tiles per SIMD (5,120 on an undivided MI355X) of small trees stay in step, more run in phases; both
+    give the single-scene image bit for bit."""
+    hs = rt.HostScene.cornell()
+    lights = rt.LightSampler(hs, 123).generate(128)
+    cam = workloads.cornell_camera(256)
+    b = rt.Batch(0)
+    try:
+        for _ in range(scenes):
+            b.add(hs, cam, 256, 256, lights, 5)
+        b.finalize()
+        print("case: batch of %d Cornell rooms" % scenes, flush=True)
+        b.draw(True)
+        single = single_scene(rt, ctx, hs, cam, 256, 256, lights, 1, rt.KERNEL_WIDE)
+        for i in range(scenes):
+            assert np.array_equal(b.readback(i).view(np.uint32), single.view(np.uint32)), i
+    finally:
+        b.close()
+
+
 def test_graph_replay_matches_eager_frames(rt):
     scenes = small_scenes(rt)
     b = rt.Batch(0)
