@@ -147,10 +147,11 @@ __device__ __forceinline__ void wide_init(const WideScene& s, WideState& st, gg:
   // A ray without a finite origin component, or with a NaN for its length, hits nothing,
   // but minima and maxima drop the NaNs of its slab distances: they would let every box
   // through.  Here the scene lies behind it, so that its walk ends at the root.
-  if (!(finite(o.x) || finite(o.y) || finite(o.z)) || tmax != tmax) {
-    st.o.x = 1e38f;
-    st.ix = s.tScale;
-  }
+  // (Selects: with a branch the compiler computes the box pass's plane selectors after
+  // the node's loads have come instead of before, 3 % for small launches.)
+  const bool dead = !(finite(o.x) || finite(o.y) || finite(o.z)) || tmax != tmax;
+  st.o.x = dead ? 1e38f : o.x;
+  st.ix = dead ? s.tScale : st.ix;
 }
 
 // The node in slot `slot` of the node whose inner children (mask `inner`) start at `first`.
