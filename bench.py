@@ -260,8 +260,8 @@ def summarize_counters(name, *dirs):
     clutter = "clutter" in name
     workload = ("clutter room, 4000 icospheres (5,120,016 triangles), 2^24 incoherent rays, closest hit"
                 if clutter else PROFILE_WORKLOAD)
-    run = ("--clutter --clutter-incoherent-only --steps 3 --calibrate --valu-probe" if clutter
-           else "--steps 2 --warmup 1 --no-cpu-baseline --calibrate --valu-probe")
+    run = ("--clutter --clutter-incoherent-only --steps 3 --calibrate" if clutter
+           else "--steps 2 --warmup 1 --no-cpu-baseline --calibrate") + (" --valu-probe" if probe else "")
     if "FETCH_SIZE" in per and "WRITE_SIZE" in per:
         gib_kib = float(1 << 20)
         fc = _pmc_per_launch([d for d in dirs if _has_counter(d, "FETCH_SIZE")][0], "FETCH_SIZE")[1]
@@ -280,7 +280,9 @@ def summarize_counters(name, *dirs):
     print(json.dumps(out))
 
 
-INTEGRATOR_KERNELS = ("k_pathtracer<true>", "k_lighttracer<true, 0>", "k_lighttracer<true, 1>", "k_bpt_eye<true>",
+INTEGRATOR_KERNELS = ("k_pathtracer_wide<false>", "k_lighttracer_wide<0, false>", "k_lighttracer_wide<1, false>",
+                      "k_bpt_eye_wide<false>", "k_pathtracer<true>", "k_lighttracer<true, 0>",
+                      "k_lighttracer<true, 1>", "k_bpt_eye<true>",
                       "k_wf_shade<0>", "k_wf_shade<1>", "k_trace_wide<false, 256, 10, false>",
                       "k_trace_wide<true, 256, 10, false>")
 
@@ -831,9 +833,10 @@ def summarize_wavefront(kt_dir):
             ds.sort()
             lines.append("  queue %s: %d launches, median %.1f us, max %.1f us" % (qid, len(ds), ds[len(ds) // 2],
                                                                                ds[-1]))
-        lines += ["A reset queued beside the other stream's persistent trace waits for a free wave slot, which",
-                  "opens only as that trace's waves exit; the trace launched behind it waits for the same slots,",
-                  "so its long durations there are queueing, not work."]
+        if any(ds[len(ds) // 2] > 100.0 for ds in resets.values()):
+            lines += ["A reset queued beside the other stream's persistent trace waits for a free wave slot, which",
+                      "opens only as that trace's waves exit; the trace launched behind it waits for the same slots,",
+                      "so its long durations there are queueing, not work."]
     for mode, title in ((0, "path-tracer"), (1, "BPT")):
         raygen = [i for i, n in enumerate(names) if n == "k_wf_raygen<%d>" % mode]
         if not raygen:
@@ -843,7 +846,7 @@ def summarize_wavefront(kt_dir):
         lines += ["", "The last wavefront %s draw, per bounce (kernel durations in us; late bounces launch over the"
                   % title, "full queue capacity and their kernels exit once the device count is reached):"]
         if mode == 1:  # the light pass that precedes the eye paths
-            lp = max(j for j in range(first) if names[j].startswith("k_lighttracer<"))
+            lp = max(j for j in range(first) if names[j].startswith(("k_lighttracer_wide<", "k_lighttracer<")))
             lines.append("  light pass (%s): %.1f us, up to the eye paths' ray generation %.2f ms" % (
                 names[lp], dur[lp], (int(rows[first]["Start_Timestamp"]) - int(rows[lp]["Start_Timestamp"])) / 1e6))
         bounce = 0

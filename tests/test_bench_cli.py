@@ -79,8 +79,8 @@ def test_integrator_counter_formulas(tmp_path, monkeypatch):
     assert set(doc["kernels"]) == {"k_pathtracer<true>"}
 
 
-@pytest.mark.parametrize("profile,kernel_ms", [("trace_wide_heightfield_pmc.json", 2.4),
-                                               ("trace_wide_clutter_pmc.json", 5.7)])
+@pytest.mark.parametrize("profile,kernel_ms", [("trace_wide_heightfield_pmc.json", 2.1),
+                                               ("trace_wide_clutter_pmc.json", 4.5)])
 def test_committed_traffic_is_a_physical_roofline_input(profile, kernel_ms):
     """The HBM traffic the bench line divides by the launch time comes from the committed
     counter summary: at least the rays read and hits written (2^24 x 48 B), and no more
