@@ -290,9 +290,9 @@ __global__ __launch_bounds__(kLightBlock) __attribute__((amdgpu_waves_per_eu(5))
 }
 
 // The same over the wide BVH, in phases (phased_paths).  Room of 4000 spheres,
-// 1920x1080, path length 8: a light-traced frame 5.21 -> 3.86 ms.  Resident blocks
-// that take new paths (a block per 64 paths: 4.04 ms); four waves per SIMD (five:
-// 3.89 ms).
+// 1920x1080, path length 8: a light-traced frame 5.21 -> 3.86 ms (3.45 with the
+// walk of today).  Resident blocks that take new paths (a block per 64 paths: 4.04
+// for those 3.86 ms); four waves per SIMD (five: 3.89).
 template <int MODE, bool WT>
 __global__ __launch_bounds__(kLightBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_lighttracer_wide(
     DrawParams p, int raysPerSample, uint32_t numPaths, LightCacheEntryDev* __restrict__ cache,

@@ -68,14 +68,16 @@ struct MlpDev {
   float* loss;       // loss partials, likewise
 };
 
-// The gradient kernel's most blocks, so partials: one per CU.
+// The gradient kernel's most blocks, so partials: one per CU of an undivided card.
+// A constant and not the device's count, since it sets the order in which the
+// gradient is summed: the same steps give the same weights on any partition.
 constexpr uint32_t kMlpGradBlocks = 256;
 // log2 of the samples in a tile of the gradient kernel, for steps of at most n
 // samples (which fixes the kernel, whatever a count on the device then says): 64
 // (eight waves) where the partials are what a step waits for, 32 (four waves)
-// where it is the chain of phases (16 steps and an inference: 0.351 -> 0.338 ms
-// for 257 samples a step, 0.427 -> 0.413 for 4,096, 0.621 -> 0.531 for 16,384; with
-// 64 below the line 0.367 for 257 and 0.372 for 1,000, which take 0.351 with 32).
+// where it is the chain of phases.  16 steps and an inference of 64 samples, in us
+// with tiles of 32 / 64 samples: 347 / 372 for 1,000 samples a step, 369 / 378 for
+// 2,048, 405 / 404 for 4,096, 485 / 442 for 8,192.
 constexpr uint32_t kMlpGradSmall = 2048;
 inline uint32_t MlpGradTileLog2(size_t n) { return n <= kMlpGradSmall ? 5u : 6u; }
 static_assert(kMlpGradSmall <= 32 * kMlpGradBlocks, "the four-wave kernel has one tile per block");

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kInferBlock) void k_mlp_infer(const uint16_t* __res
 // k_mlp_reduce) and by the chain of ten phases.  Eight waves halve the partials,
 // and a block keeps its partial in registers over its tiles, so that there are
 // at most kMlpGradBlocks (20 MB) for any batch: 16 Adam steps and an inference of
-// 64 samples take 0.614 -> 0.531 ms for 16,384 samples a step and 1.42 -> 0.98 ms
+// 64 samples take 0.614 -> 0.525 ms for 16,384 samples a step and 1.42 -> 0.98 ms
 // for 65,536, against one partial per 32-sample tile (40 and 160 MB each way).
 // One block of eight waves per CU (138 KB of LDS).  Four waves (MlpGradTileLog2)
 // run one tile per block.

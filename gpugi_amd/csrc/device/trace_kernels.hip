@@ -185,7 +185,7 @@ hipError_t LaunchTraceRef(const RefScene& s, int query, const gpugi_ray* rays, g
   // with resident waves).  Else at most eight blocks per CU, which hide the loads'
   // latency best, or six where each still gets four batches and more and the tree is
   // larger than an XCD's L2 (4 MB): fewer waves share the L1 better (2^23 diffuse rays,
-  // 2,097,152-triangle heightfield: 3.1 against 3.4 ms).  Whole blocks per XCD.
+  // 2,097,152-triangle heightfield: 3.3 against 3.5 ms).  Whole blocks per XCD.
   const uint32_t batches = (uint32_t)((n + 63) / 64);
   const uint32_t perX = (batches + kRefXcds - 1) / kRefXcds;
   const uint32_t resident = (uint32_t)cus * 8 * kRefWaves, blocks = (perX + kRefWaves - 1) / kRefWaves;

@@ -20,14 +20,14 @@
 // cap the waves per CU (160 KiB LDS per CU); the autotuner picks it.
 //
 // Bound by VALU issue (1.13 wave-instructions per CU and cycle, an FMA stream
-// reaches 0.99) and by the vector-memory data path (TD busy 94 % of the cycles)
+// reaches 0.99) and by the vector-memory data path (TD busy 93 % of the cycles)
 // at once, so a node holds eight children in five 16-byte loads: against
 // four-child nodes of four loads, 0.67 times the node visits and about the
 // same instructions per visit.  Measured (2^24 diffuse rays, 2,097,152-triangle
 // heightfield; 2^22 camera / diffuse / shadow rays, 5,120,016-triangle room):
-// four children 2471 us; 3054 / 1889 / 1193 us; eight 2194; 1526 / 1413 / 953 us.
-// Seven waves per SIMD (72 VGPRs, no spill): six measured 2282 us on the
-// heightfield set, eight spill 44 bytes a lane in the box pass and take 3248 us.
+// four children 2495 us; 2769 / 1797 / 1143 us; eight 2139; 1252 / 1338 / 1004 us.
+// Seven waves per SIMD (72 VGPRs, no spill).  Six took 1.04 times as long on the
+// heightfield set, eight, which spill 44 bytes a lane in the box pass, 1.48 times.
 // Compiled with -ffp-contract=off: the triangle test must round exactly like
 // the reference formula.
 #include <hip/hip_runtime.h>
