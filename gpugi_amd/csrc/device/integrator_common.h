@@ -123,12 +123,12 @@ struct QueueChunks {
 // does not depend on when its passes run.  Items come in chunks of `lanes` from
 // `source`; the first `lanes` lanes of the wave carry them.
 //
-// Bound by VALU issue (1.0 wave-instructions per CU and cycle).  Against tracing
-// each ray where it is needed (persistent_items), whose passes run with the
-// lanes of every other phase masked off: 35 lanes active instead of 16, path
-// tracing the 5,120,016-triangle room at 1920x1080 (path length 8) 9.5 -> 6.5 ms
-// a frame.  Four waves per SIMD (128 VGPRs): five spill 112 bytes a lane and
-// take 6.6 ms.
+// Bound by VALU issue (0.92 wave-instructions per CU and cycle) and the L1's data
+// path (TD busy 89 %).  Against tracing each ray where it is needed
+// (persistent_items), whose passes run with the lanes of every other phase masked
+// off: 25 lanes active instead of 18, path tracing the 5,120,016-triangle room at
+// 1920x1080 (path length 8) 9.5 -> 6.5 ms a frame.  Four waves per SIMD (128 VGPRs):
+// five spill 112 bytes a lane and take 6.6 ms.
 template <bool WT, int S, class Source, class Prog>
 __device__ __forceinline__ void phased_paths(const WideScene& ws, uint2* lds, uint2* spill, uint32_t numItems,
                                              Source& source, uint32_t lanes, Prog& prog) {
